@@ -102,8 +102,10 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
  * (no initial contents needed): 17..64 rows on large matrices (and from 4
  * rows where the decode kernels have no good layout for x, e.g. K = 11008
  * at 15-16 rows; a smaller workspace is refused for these), and prefill
- * calls whose row tiles make at most one round of the GPU (a smaller
- * workspace runs those unsplit); other sizes need none (0).  Calls that
+ * calls, also those of 17..64 rows with zero points or fp32 scales, whose
+ * estimated time a K split shortens (a smaller workspace runs those
+ * unsplit, or on the decode kernels); other sizes need none (0).  A split
+ * keeps rows of N rounded up to a multiple of 4.  Calls that
  * overlap in time must not share a workspace. */
 size_t zt_woq_linear_workspace_size(int64_t M, int64_t K, int64_t N,
                                     int64_t G);

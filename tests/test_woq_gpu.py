@@ -710,3 +710,44 @@ def test_lean_kernel_gate_up(M, K, I, G, form, knobs):
     knobs.set("ZT_WOQ_LEAN", "0")
     y_other, _ = run_gate_up(M, K, I, G, seed=M + I + 2)
     check_close(y, y_other.cpu())
+
+
+# the large-tile prefill kernel: every tile, K splits, groups of 32 and up,
+# ragged M and N (rows that are not whole quads too), one step of K, and each
+# dequantisation (signed; 8-bit zero points; other zero points and fp32 scales)
+@pytest.mark.parametrize("tile", ["p0", "p1", "p2", "p03", "p12", "p23"])
+@pytest.mark.parametrize("zp,s_dtype", [(None, torch.bfloat16), (torch.int8, torch.bfloat16),
+                                        (torch.uint8, torch.bfloat16), ("int", torch.float32),
+                                        ("float", torch.bfloat16)])
+@pytest.mark.parametrize("M,K,N,gs", [(1, 64, 20, 32), (257, 832, 517, 64), (130, 1024, 258, 128),
+                                      (300, 960, 131, 960)])
+def test_prefill_kernel_vs_oracle(M, K, N, gs, zp, s_dtype, tile, knobs):
+    knobs.set("ZT_WOQ_FORCE_KERNEL", "gemm")
+    knobs.set("ZT_WOQ_GEMM", tile)
+    as_int = isinstance(zp, torch.dtype)
+    x, q, wp, s, z, b = make_case(M, K, N, K // gs, M + N, zp="int" if as_int else zp, bias=True,
+                                  s_dtype=s_dtype)
+    z = z.to(zp) if as_int else z
+    res = torch.randn(M, N, generator=torch.Generator().manual_seed(3)).bfloat16()
+    y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b, post_ops=("silu", "mul"), post_bufs=[res])
+    xd, wd, sd, zd, bd = gpu(x, wp, s, z, b)
+    y = C.woq_linear(xd, wd, sd, zd, bd, post_ops=("silu", "mul"), post_bufs=gpu(res))
+    check_close(y, y_ref)
+
+
+@pytest.mark.parametrize("tile", ["p0", "p1", "p2"])
+@pytest.mark.parametrize("M,K,I,gs,zp", [(65, 128, 33, 32, None), (300, 512, 200, 64, "int"),
+                                         (129, 256, 128, 128, "float")])
+def test_prefill_kernel_gate_up(M, K, I, gs, zp, tile, knobs):
+    knobs.set("ZT_WOQ_GEMM", tile)
+    run_gate_up(M, K, I, K // gs, seed=M + I, zp=zp)
+
+
+# zero points at 17..64 rows: the prefill kernel when the workspace holds its
+# splits
+@pytest.mark.parametrize("M,K,N", [(17, 4096, 520), (64, 2048, 261)])
+def test_zero_points_17_to_64_rows(M, K, N, knobs, capfd):
+    knobs.set("ZT_WOQ_DEBUG", "1")
+    capfd.readouterr()
+    run_case(M, K, N, K // 128, zp="int", seed=M + N, bias=True)
+    assert "woq prefill" in capfd.readouterr().err

@@ -280,7 +280,7 @@ size_t zt_woq_linear_workspace_size(int64_t M, int64_t K, int64_t N,
   a.w = reinterpret_cast<const uint32_t *>(256);
   // the prefill GEMM's K-split partials (few tiles)
   const size_t gemm = zt::woq_gemm_workspace(M, N, K);
-  if (zt::woq_select_kernel(a) != zt::kWoqDecode) return std::max(wide, gemm);
+  if (M > kWoqRowBlock || zt::woq_select_kernel(a) != zt::kWoqDecode) return std::max(wide, gemm);
   zt::DecodePlan p;
   if (!zt::woq_decode_plan(M, N, K, &p)) return std::max(wide, gemm);
   return std::max(wide, zt::woq_decode_workspace(p, M, N));
@@ -346,6 +346,17 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
                   workspace ? workspace_bytes : (size_t)0);
     return hip_status(zt::launch_woq_wide(a, wp, workspace, s), op);
   }
+  // 17..64 rows with zero points or fp32 scales, which the wide kernel does
+  // not take: the prefill GEMM, K split over the workspace, reads the weights
+  // once where the decode kernels' general modes pay their longer
+  // dequantisation per row block (zero points, 24 / 64 rows: 4096 x 4096 17.8 /
+  // 34.6 -> 16.8 / 21.2 us, 18944 x 3584 68.7 / 167 -> 31.0 / 35.1,
+  // 3584 x 18944 62.4 / 131 -> 33.5 / 37.1)
+  if (M > kWoqRowBlock && M <= kWoqRowBlockMax && (zp || scales_dtype == ZT_DT_F32) &&
+      !zt::knob(zt::kKnobWoqForceKernel) && !zt::knob(zt::kKnobWoqStream) &&
+      zt::woq_prefill_ok(a) && workspace &&
+      workspace_bytes >= zt::woq_prefill_workspace(M, N, K))
+    return hip_status(zt::launch_woq_prefill(a, false, workspace, workspace_bytes, s), op);
   if (woq_use_row_blocks(a)) {
     // one stream-kernel launch over all rows when x (in K phases) fits, else
     // blocks of 16 rows
@@ -407,6 +418,9 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   hipError_t err = hipSuccess;
   if (zt::woq_try_stream_gate_up(a, s, &err)) return hip_status(err, op);
   if (zt::woq_try_wide_gate_up(a, s, &err)) return hip_status(err, op);
+  const char *forced = zt::knob(zt::kKnobWoqGemm);
+  if ((!forced || forced[0] == 'p') && zt::woq_prefill_ok(a))
+    return hip_status(zt::launch_woq_prefill(a, true, nullptr, 0, s), op);
   // two steps: the full [M, N] linear in fp32 into the workspace, then
   // silu(gate) * up over its halves
   const size_t h = ((size_t)M * (size_t)N * sizeof(float) + 255) / 256 * 256;

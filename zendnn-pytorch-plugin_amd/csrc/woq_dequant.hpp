@@ -59,6 +59,26 @@ __device__ __forceinline__ u32x4_t dq8_s4_bf16scale(uint32_t w, float s, float s
   return r;
 }
 
+// Unsigned int4 with a bf16 scale s and an 8-bit integer zero point z:
+//   fma(1024 + u,   s,    -(1024 + z) s) = (u - z) s
+//   fma(1024 + 16u, s/16, -(64 + z) s)   = (u - z) s
+// exact as above: 1024 + z and 64 + z have at most 11 significant bits, so
+// their products with s at most 19, and (u - z) s at most 17.
+__device__ __forceinline__ u32x4_t dq8_u4_bf16scale(uint32_t w, float s, float z) {
+  const uint32_t w8 = w >> 8;
+  const uint32_t p0 = and_xor(w, kNibLo, kExpLo);
+  const uint32_t p1 = and_xor(w, kNibHi, kExpLo);
+  const uint32_t p2 = and_xor(w8, kNibLo, kExpLo);
+  const uint32_t p3 = and_xor(w8, kNibHi, kExpLo);
+  const float s16 = s * 0.0625f, c0 = -(1024.f + z) * s, c1 = -(64.f + z) * s;
+  u32x4_t r;
+  r[0] = pack_bf16x2(fmaf(f16_lo(p0), s, c0), fmaf(f16_lo(p1), s16, c1));
+  r[1] = pack_bf16x2(fmaf(f16_lo(p2), s, c0), fmaf(f16_lo(p3), s16, c1));
+  r[2] = pack_bf16x2(fmaf(f16_hi(p0), s, c0), fmaf(f16_hi(p1), s16, c1));
+  r[3] = pack_bf16x2(fmaf(f16_hi(p2), s, c0), fmaf(f16_hi(p3), s16, c1));
+  return r;
+}
+
 // Per-(row, group) constants of the general path.
 struct DqGeneral {
   uint32_t xlo, xhi;  // XOR bits (signed int4) or 0 (unsigned)

@@ -29,12 +29,15 @@
 //    x in registers and the next units' weights in flight.
 //  * woq_decode_kernel   the older decode kernel for shapes the two above do
 //    not take (long K split over workgroups, general dequant modes).
-//  * woq_gemm32_kernel / woq_gemm_ws_kernel / woq_gemm_dma_kernel  prefill
-//    (more rows): LDS tiles moved by DMA, int4 dequantised in registers
-//    after the LDS read, bf16 MFMA (32x32x16 for signed int4 with bf16
-//    scales -- with load waves of their own when one round of tiles covers
-//    the matrix -- 16x16x32 for the other modes); woq_gemm_kernel for group
-//    sizes that are not multiples of 128.
+//  * woq_prefill_kernel (woq_prefill.hip)  more rows than the decode kernels
+//    take, groups of 32 and up, any zero-point and scale type; also 17..64
+//    rows with zero points or fp32 scales, and any row count in groups of 32
+//    and 64.
+//  * woq_gemm_ws_kernel  one nearly full round of 256 x 128 tiles at up to
+//    512 rows (signed int4, bf16 scales): loads in waves of their own, three
+//    stages.  woq_gemm32_kernel / woq_gemm_dma_kernel / woq_gemm_kernel: the
+//    kernels before woq_prefill_kernel, selectable, and for what its 32-bit
+//    offsets and group sizes exclude.
 //  * woq_generic_kernel  what none of the above takes (K not a multiple of
 //    64, odd group sizes): one wave per output element.
 //
@@ -3023,7 +3026,8 @@ int woq_gemm_splits(int64_t M, int64_t N, int64_t K) {
 
 size_t woq_gemm_workspace(int64_t M, int64_t N, int64_t K) {
   const int sp = woq_gemm_splits(M, N, K);
-  return sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : 0;
+  return std::max(sp > 1 ? (size_t)sp * (size_t)M * (size_t)N * sizeof(float) : (size_t)0,
+                  woq_prefill_workspace(M, N, K));
 }
 
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {
@@ -3031,6 +3035,18 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace, size_t workspace_bytes) {
+  const char *forced = knob(kKnobWoqGemm);
+  // The large-tile kernel, except where the load-wave kernel below is still
+  // ahead: one round of its 256 x 128 tiles at least three quarters full over
+  // at most two row tiles, where the weights come from HBM and its third
+  // stage hides more of that (signed int4 with bf16 scales; 28672 x 4096 at
+  // M = 256 70.4 against 73-77 us, 16384 x 3072 at M = 512 57 against 60).
+  const int64_t lw_tiles = ((a.M + 255) / 256) * ((a.N + 127) / 128);
+  const bool load_wave = a.M <= 512 && lw_tiles > 192 && lw_tiles <= 256 && !a.zp &&
+                         a.s_dt == ZT_DT_BF16 && a.N % 8 == 0 && a.K % 128 == 0 &&
+                         (a.G == 1 || (a.K / a.G) % 128 == 0);
+  if (a.M > 0 && a.N > 0 && (forced ? forced[0] == 'p' : !load_wave) && woq_prefill_ok(a))
+    return launch_woq_prefill(a, false, workspace, workspace_bytes, s);
   {
     // the DMA kernel: bf16 x, K % 128 == 0, one scale per 128-chunk, 32-bit
     // byte offsets for x and the weights

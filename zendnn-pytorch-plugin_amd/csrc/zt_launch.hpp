@@ -56,6 +56,20 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s);
 // with less it runs unsplit.
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace,
                            size_t workspace_bytes);
+// Large-tile prefill GEMM (woq_prefill.hip): whether it takes these
+// operands, the tile and K split it takes for a shape (tile 0: 128 x 128, 1:
+// 128 x 256, 2: 256 x 256; us: the estimate they were chosen by), the bytes of
+// the splits' fp32 partials (0: none; given less it runs unsplit), and the
+// whole call (gate_up: the merged silu(gate) * up form, never split).
+struct PrefillPlan {
+  int tile = -1, splits = 1;
+  double us = 0;
+};
+bool woq_prefill_ok(const WoqArgs &a);
+PrefillPlan woq_prefill_plan(int64_t M, int64_t N, int64_t K, bool gate_up);
+size_t woq_prefill_workspace(int64_t M, int64_t N, int64_t K);
+hipError_t launch_woq_prefill(const WoqArgs &a, bool gate_up, void *workspace,
+                              size_t workspace_bytes, hipStream_t s);
 int woq_gemm_splits(int64_t M, int64_t N, int64_t K);
 size_t woq_gemm_workspace(int64_t M, int64_t N, int64_t K);
 // The weight-streaming decode kernel for up to 64 rows, when it applies
