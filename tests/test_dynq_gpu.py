@@ -370,3 +370,31 @@ def test_s8_large_m_kernels_bit_exact(kind, M, N, K, knobs):
     y = C.dynamic_qlinear(x.to(DEV), w2.to(DEV), sw.to(DEV), b.to(DEV)).cpu()
     torch.testing.assert_close(y.float(), O.dynamic_qlinear(x, w2, sw, b).float(), rtol=1e-2,
                                atol=1e-2)
+
+
+# the 256 x 256 kernel (ZT_S8_KIND p): ragged M and N (rows that are not
+# whole quads too), K of one, two and an odd number of steps and not a
+# multiple of the step; raw sums, symmetric and asymmetric activations,
+# post-ops and fp32 outputs, against the oracle and the kernels before it
+@pytest.mark.parametrize("M,N,K", [(129, 20, 16), (257, 517, 272), (300, 258, 384), (520, 131, 128)])
+@pytest.mark.parametrize("kind", ["p", "w"])
+def test_s8_256_tile_kernel(kind, M, N, K, knobs):
+    knobs.set("ZT_S8_KIND", kind)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-128, 128, (M, K), generator=g, dtype=torch.int8)
+    w8 = torch.randint(-128, 128, (N, K), generator=g, dtype=torch.int8)
+    assert torch.equal(C.s8s8s32_gemm(a.to(DEV), w8.to(DEV)).cpu(), a.int() @ w8.t().int())
+    for x_dtype, post in [(torch.bfloat16, ()), (torch.bfloat16, ("add",)),
+                          (torch.float32, ("silu", "mul")), (torch.bfloat16, ("mul", "add"))]:
+        x, w, sw, b = make(M, K, N, seed=M + K, x_dtype=x_dtype)
+        bufs = [torch.randn(M, N, generator=g).to(x_dtype) for p in post if p in ("add", "mul")]
+        args = (x.to(DEV), w.to(DEV), sw.to(DEV), b.to(DEV))
+        y = C.dynamic_qlinear(*args, post_ops=post, post_bufs=[t.to(DEV) for t in bufs]).cpu()
+        y_ref = O.dynamic_qlinear(x, w, sw, b, post_ops=post, post_bufs=bufs)
+        tol = 1e-2 if x_dtype == torch.bfloat16 else 1e-4
+        torch.testing.assert_close(y.float(), y_ref.float(), rtol=tol, atol=tol)
+    colsum = C.s8_weight_colsum(w.to(DEV))
+    acc = C.dynamic_qlinear_asym(x.to(DEV), w.to(DEV), sw.to(DEV), colsum, None,
+                                 out_dtype=torch.int32).cpu()
+    q, _, zp = O.dynamic_quantize_asym(x)
+    assert torch.equal(acc, (q.int() - zp[:, None].int()) @ w.t().int())

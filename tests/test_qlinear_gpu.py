@@ -184,3 +184,18 @@ def test_qlinear_weight_column_sums_cached_and_updated():
     wd3 = w3.to(DEV)
     check(call(wd3), O.qlinear(x, w3, xs, xz, ws, b, out_dtype=torch.float32))
     assert wd3.data_ptr() == ptr or True  # the caching allocator usually reuses the block
+
+
+# requantised outputs, with and without a post-op, from the 256 x 256 kernel
+# and from the load-wave kernel's tile epilogue
+@pytest.mark.parametrize("kind", ["p", "w"])
+@pytest.mark.parametrize("N", [264, 131])
+@pytest.mark.parametrize("post", [[], ["relu"]])
+def test_qlinear_requantised_large_m(kind, N, post, knobs):
+    knobs.set("ZT_S8_KIND", kind)
+    x, w, xs, xz, ws, b = make(N, shape=(300, 400), N=N, in_dtype=torch.bfloat16)
+    ys, yz = torch.tensor([0.7]), torch.tensor([90], dtype=torch.int32)
+    op = ops.zentorch_qlinear_relu if post else ops.zentorch_qlinear
+    y = op(*dev(x, w, xs, xz, ws, None, b, ys, yz), output_dtype=torch.uint8)
+    check(y, O.qlinear(x, w, xs, xz, ws, b, post_ops=post, out_dtype=torch.uint8, y_scale=ys,
+                       y_zp=yz))

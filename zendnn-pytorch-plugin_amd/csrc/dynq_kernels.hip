@@ -21,6 +21,7 @@
 #include <cstdio>
 #include <cstdlib>
 
+#include "s8_epilogue.hpp"
 #include "zt_launch.hpp"
 #include "zt_tuning.hpp"
 
@@ -469,6 +470,40 @@ __device__ __forceinline__ void s8_tile_epilogue(const DynArgs &a, const int32_t
       }
     }
     return;
+  }
+  // Post-ops and requantised outputs, when whole passes of rows cover the
+  // tile: scaled in place, the post-ops one by one over the tile (their binary
+  // operands' loads in flight together), then stored.  Quad by quad
+  // (below) each one waited for its own scales and operands: 3000 x 4096 x 1024
+  // to u8 129 us in all against 25, a silu * mul at 4096 x 4096 x 4096 174
+  // against 92 without.
+  constexpr int RP = NTE / G4, T = BM / RP;
+  if constexpr (T * RP == BM && T <= 16) {
+    if (a.y_dt != ZT_DT_S32) {
+      if (n >= N || tid >= NTE) return;
+      QuadScales qs;
+      qs.load(a, n, N);
+      int32_t *rows = const_cast<int32_t *>(tile);
+      float *frows = reinterpret_cast<float *>(rows);
+      const int r0 = tid / G4;
+#pragma unroll 4
+      for (int t = 0; t < T; ++t) {
+        const int row = t * RP + r0;
+        const i32x4_t v = *reinterpret_cast<const i32x4_t *>(rows + row * AP + c4);
+        float f[4];
+        qs.scale(qs.correct(v, a.azp ? a.azp[min(m0 + row, M - 1)] : 0), sx_l[row], f);
+        *reinterpret_cast<f32x4_t *>(frows + row * AP + c4) = f32x4_t{f[0], f[1], f[2], f[3]};
+      }
+      post_ops_slab<T, RP>(frows, AP, c4, r0, a.post, m0, n, M, N);
+#pragma unroll 4
+      for (int t = 0; t < T; ++t) {
+        const int row = t * RP + r0;
+        const f32x4_t v = *reinterpret_cast<const f32x4_t *>(frows + row * AP + c4);
+        const float f[4] = {v[0], v[1], v[2], v[3]};
+        if (m0 + row < M) store_y4(a, qs, m0 + row, n, N, f);
+      }
+      return;
+    }
   }
   for (int idx = tid; idx < BM * G4; idx += NT) {
     const int row = idx / G4, cc = (idx % G4) * 4;
@@ -2210,7 +2245,8 @@ hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s) {
     const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 127) / 128);
     const char *tile = knob(kKnobS8Tile);
     const bool big = tile ? tile[0] == '2' : t256 >= 128;
-    const char *kind = knob(kKnobS8Kind);  // w: load-wave kernel, n: 32x32x32 kernel, r, 2, 3
+    const char *kind = knob(kKnobS8Kind);  // p: large tiles, w: load waves, n: 32x32x32 kernel, r, 2, 3
+    if (!tile && kind && kind[0] == 'p') return launch_s8_prefill(a, s);
     if (!kind || kind[0] == 'w') {
       // ZT_S8_TILE: "2" 256 x 128 tiles, "1" 128 x 128 with 3 stages, "0" 128 x 128 with 2
       // stages (two workgroups per CU)
@@ -2234,6 +2270,7 @@ hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s) {
       // 256 x 192 tiles (six compute waves of 128 x 64, two load waves, two
       // stages) where they make one round and 256 x 128 tiles do not: QKV at
       // M = 2048, 256 against 384 tiles, 69 -> 58.5 us
+      if (!tile && !kind && s8_prefill_better(a.M, a.N, a.K)) return launch_s8_prefill(a, s);
       const int64_t t192 = ((a.M + 255) / 256) * ((a.N + 191) / 192);
       const bool w192 = tile ? tile[0] == '9' : t256 > 256 && t192 <= 256;
       if (w192) return launch_s8_ws<256, 192, 2, 3, 2, 2>(a, s);

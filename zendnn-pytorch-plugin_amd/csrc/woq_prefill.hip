@@ -259,6 +259,20 @@ void woq_prefill_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int gs
   // 8- or 16-bit values it would extend them, and wait, at its top)
   asm volatile("" : "+v"(qnext.s), "+v"(qnext.z));
   dma(kb + 1, 1);
+  // the epilogue's columns and their bias, loaded ahead of the main loop
+  constexpr int SP = 64 + 4;            // slab pitch, floats
+  constexpr int Q = GU ? 8 : 16;        // column quads of y per wave and row
+  constexpr int RP = 64 / Q;            // rows per pass
+  const int c4 = (lane % Q) * 4, r0 = lane / Q;
+  const int n = n0 + wn * 4 * Q + c4;
+  float bias[4] = {0.f, 0.f, 0.f, 0.f}, ubias[4] = {0.f, 0.f, 0.f, 0.f};
+  if (a.bias && !partial)
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+      if (n + r < NY) {
+        bias[r] = load_elem(a.bias, a.b_dt, n + r);
+        if (GU) ubias[r] = load_elem(a.bias, a.b_dt, NY + n + r);
+      }
   read(smem, 0, 0);
   int cur = 0;
   for (int ks = kb; ks < ke; ++ks, cur ^= 1) {
@@ -298,21 +312,7 @@ void woq_prefill_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int gs
   // m = l % 32; the slab turns it into rows of four columns per lane).  The
   // loops stay rolled: the code runs once per tile, and unrolled its
   // instruction fetches alone took 30 us.
-  constexpr int SP = 64 + 4;            // slab pitch, floats
-  constexpr int Q = GU ? 8 : 16;        // column quads of y per wave and row
-  constexpr int RP = 64 / Q;            // rows per pass
   float *slab = reinterpret_cast<float *>(smem) + wv * (32 * SP);
-  const int c4 = (lane % Q) * 4, r0 = lane / Q;
-  const int n = n0 + wn * 4 * Q + c4;
-  const bool plain = !GU && !partial && !a.post.count;
-  float bias[4] = {0.f, 0.f, 0.f, 0.f}, ubias[4] = {0.f, 0.f, 0.f, 0.f};
-  if (a.bias && !partial)
-#pragma unroll
-    for (int r = 0; r < 4; ++r)
-      if (n + r < NY) {
-        bias[r] = load_elem(a.bias, a.b_dt, n + r);
-        if (GU) ubias[r] = load_elem(a.bias, a.b_dt, NY + n + r);
-      }
   const bool has_bias = a.bias != nullptr;
 #pragma unroll 1
   for (int i = 0; i < TM; ++i) {
@@ -328,43 +328,46 @@ void woq_prefill_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int gs
                         acc[ii][j][4 * r + 3]};
     __builtin_amdgcn_wave_barrier();
     const int mb = m0 + wm * (BM / WM) + i * 32;
-    if (plain) {
+    if (GU || (a.post.count && !partial)) {
+#pragma unroll 1
+      for (int t = 0; t < 32 / RP; ++t) {
+        float *at = slab + (t * RP + r0) * SP + c4;
+        f32x4_t v = *reinterpret_cast<const f32x4_t *>(at);
+        if (GU) {
+          const f32x4_t u = *reinterpret_cast<const f32x4_t *>(at + 32);
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const float g = has_bias ? v[r] + bias[r] : v[r];
+            float up = has_bias ? u[r] + ubias[r] : u[r];
+            if (a.y_dt == ZT_DT_BF16) up = bf16_bits_to_f32(f32_to_bf16_bits(up));
+            v[r] = unary_op(ZT_PO_SILU, g) * up;
+          }
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = has_bias ? v[r] + bias[r] : v[r];
+        }
+        *reinterpret_cast<f32x4_t *>(at) = v;
+      }
+      if (!GU) post_ops_slab<32 / RP, RP>(slab, SP, c4, r0, a.post, mb, n, M, N);
+    }
+    if (partial) {  // rows of whole quads
+#pragma unroll 4
+      for (int t = 0; t < 32 / RP; ++t) {
+        const int row = t * RP + r0, m = mb + row;
+        if (m < M && n < N)
+          *reinterpret_cast<f32x4_t *>(partial + ((size_t)blockIdx.y * M + m) * pf_pitch(N) + n) =
+              *reinterpret_cast<const f32x4_t *>(slab + row * SP + c4);
+      }
+    } else {
+      const bool add = has_bias && !GU && !a.post.count;
 #pragma unroll 4
       for (int t = 0; t < 32 / RP; ++t) {
         const int row = t * RP + r0, m = mb + row;
         const f32x4_t v = *reinterpret_cast<const f32x4_t *>(slab + row * SP + c4);
         float f[4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) f[r] = has_bias ? v[r] + bias[r] : v[r];
-        if (m < M && n < N) store4(a.y, a.y_dt, a.ldy, m, n, N, f);
-      }
-    } else {
-#pragma unroll 1
-      for (int t = 0; t < 32 / RP; ++t) {
-        const int row = t * RP + r0, m = mb + row;
-        const f32x4_t v = *reinterpret_cast<const f32x4_t *>(slab + row * SP + c4);
-        float f[4];
-        if (GU) {
-          const f32x4_t u = *reinterpret_cast<const f32x4_t *>(slab + row * SP + 32 + c4);
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const float g = has_bias ? v[r] + bias[r] : v[r];
-            float up = has_bias ? u[r] + ubias[r] : u[r];
-            if (a.y_dt == ZT_DT_BF16) up = bf16_bits_to_f32(f32_to_bf16_bits(up));
-            f[r] = unary_op(ZT_PO_SILU, g) * up;
-          }
-        }
-        if (m >= M || n >= NY) continue;
-        if (!GU) {
-          if (partial) {  // rows of whole quads
-            *reinterpret_cast<f32x4_t *>(partial + ((size_t)blockIdx.y * M + m) * pf_pitch(N) + n) = v;
-            continue;
-          }
-#pragma unroll
-          for (int r = 0; r < 4; ++r) f[r] = has_bias ? v[r] + bias[r] : v[r];
-          post_ops4(f, a.post, m, n, N);
-        }
-        store4(a.y, a.y_dt, a.ldy, m, n, NY, f);
+        for (int r = 0; r < 4; ++r) f[r] = add ? v[r] + bias[r] : v[r];
+        if (m < M && n < NY) store4(a.y, a.y_dt, a.ldy, m, n, NY, f);
       }
     }
     __builtin_amdgcn_wave_barrier();

@@ -37,11 +37,17 @@ __device__ __forceinline__ void dma16(i32x4_t rsrc, uint32_t lds, uint32_t voff,
                : "memory");
 }
 
-// All of this wave's loads and LDS accesses done, then the workgroup barrier.
-__device__ __forceinline__ void wait_step() {
-  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+// At most N of this wave's loads outstanding (they retire in order) and its
+// LDS accesses done, then the workgroup barrier.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  static_assert(N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | 0x0070);
   asm volatile("s_barrier" ::: "memory");
 }
+
+// All of this wave's loads and LDS accesses done, then the workgroup barrier.
+__device__ __forceinline__ void wait_step() { wait_loads<0>(); }
 
 // Tile (tm, tn) of workgroup b: groups of group_m row tiles walked column by
 // column, each XCD on one contiguous range of that order.
@@ -91,6 +97,63 @@ __device__ __forceinline__ void post_ops4(float (&f)[4], const PostOps &p, int64
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r) f[r] = unary_op(id, f[r]);
+    }
+  }
+}
+
+// Post-ops over a wave's 32-row slab of fp32 results in LDS, in place: lane
+// holds column quads c4 of rows r0 + t * RP (t < T), global row mb + that and
+// column n.  Op by op over the whole slab and not quad by quad: the binary
+// operands of all T rows are then in flight together (a quad at a time each
+// waited for its own load, 32 round trips per tile), and the unary functions'
+// code exists once.
+template <int T, int RP>
+__device__ __forceinline__ void post_ops_slab(float *slab, int pitch, int c4, int r0,
+                                              const PostOps &p, int mb, int n, int M, int N) {
+  int b = 0;
+  for (int i = 0; i < p.count; ++i) {
+    const int id = p.ids[i];
+    if (id == ZT_PO_ADD || id == ZT_PO_MUL) {
+      const bool f32 = p.dts[b] == ZT_DT_F32;
+      const int es = f32 ? 4 : 2;
+      const char *base = static_cast<const char *>(p.bufs[b]) + (int64_t)n * es;
+      const int64_t ld = p.ld[b] * es;
+      const bool vec = n + 3 < N && !f32 && ((reinterpret_cast<uintptr_t>(base) | ld) & 7) == 0;
+      if (vec) {
+        u32x2_t o[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+          o[t] = *reinterpret_cast<const u32x2_t *>(base + min(mb + t * RP + r0, M - 1) * ld);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          f32x4_t *q = reinterpret_cast<f32x4_t *>(slab + (t * RP + r0) * pitch + c4);
+          const f32x4_t w = {bf16_bits_to_f32(o[t][0] & 0xffffu), __uint_as_float(o[t][0] & 0xffff0000u),
+                             bf16_bits_to_f32(o[t][1] & 0xffffu), __uint_as_float(o[t][1] & 0xffff0000u)};
+          *q = id == ZT_PO_ADD ? *q + w : *q * w;
+        }
+      } else {
+#pragma unroll 1
+        for (int t = 0; t < T; ++t) {
+          float *q = slab + (t * RP + r0) * pitch + c4;
+          const int64_t at = min(mb + t * RP + r0, M - 1) * p.ld[b] + n;
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (n + r < N) {
+              const float w = load_elem(p.bufs[b], p.dts[b], at + r);
+              q[r] = id == ZT_PO_ADD ? q[r] + w : q[r] * w;
+            }
+        }
+      }
+      ++b;
+    } else {
+#pragma unroll 1
+      for (int t = 0; t < T; ++t) {
+        f32x4_t *q = reinterpret_cast<f32x4_t *>(slab + (t * RP + r0) * pitch + c4);
+        f32x4_t v = *q;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = unary_op(id, v[r]);
+        *q = v;
+      }
     }
   }
 }

@@ -162,6 +162,11 @@ size_t s8_split_bytes(int64_t M, int64_t K, int64_t N);
 // K splits of the tiled int8 GEMM past 128 tokens when its 128 x 128 tiles
 // make less than one round (1 = none)
 int s8_ws_splits(int64_t M, int64_t N, int64_t K);
+// Large-tile int8 GEMM (s8_prefill.hip; qx and w 16-byte aligned, K % 16 ==
+// 0, 32-bit byte offsets): whether its 256 x 256 tiles are estimated faster
+// than 256 x 128 ones on s8_gemm_ws_kernel, and the launch.
+bool s8_prefill_better(int64_t M, int64_t N, int64_t K);
+hipError_t launch_s8_prefill(const DynArgs &a, hipStream_t s);
 int s8_split_counters(int64_t N);
 hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s);
 // The 16-token skinny GEMM with the per-token quantisation in its prologue
