@@ -81,18 +81,22 @@ __device__ __forceinline__ int quant_one(float x, float s, float inv, float zp) 
   return (int)fminf(fmaxf(r, -128.f), 127.f);
 }
 
-// Reduce (lo, hi) over the 256 threads; returns the workgroup's values.
+// Reduce (lo, hi) over the NT threads (red: NT / 32 floats); returns the
+// workgroup's values.
+template <int NT = 256>
 __device__ __forceinline__ void block_minmax(float &lo, float &hi, float *red, int tid) {
+  constexpr int NW = NT / 64;
   const int lane = tid & 63, wv = tid >> 6;
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
     lo = fminf(lo, __shfl_xor(lo, off, kWave));
     hi = fmaxf(hi, __shfl_xor(hi, off, kWave));
   }
-  if (lane == 0) red[wv] = lo, red[4 + wv] = hi;
+  if (lane == 0) red[wv] = lo, red[NW + wv] = hi;
   __syncthreads();
-  lo = fminf(fminf(red[0], red[1]), fminf(red[2], red[3]));
-  hi = fmaxf(fmaxf(red[4], red[5]), fmaxf(red[6], red[7]));
+  lo = red[0], hi = red[NW];
+#pragma unroll
+  for (int w = 1; w < NW; ++w) lo = fminf(lo, red[w]), hi = fmaxf(hi, red[NW + w]);
 }
 
 // The quantise kernels also clear the tile counters of the split-K GEMM that
@@ -134,32 +138,52 @@ __global__ __launch_bounds__(256) void dyn_quantize_kernel(
         (int8_t)quant_one<ASYM>(load_elem(x, x_dt, base + k), s, inv, zp);
 }
 
-// The same per-row quantisation for bf16 rows with K % 8 == 0, 16-byte
-// aligned: each thread holds up to VPT 8-element vectors of its row in
-// registers between the amax and the quantise pass and writes 8 bytes of qx
-// at a time (row-major, or in fragment order when FRAG).  Bit-identical to
+// Eight elements of a bf16 (one 16-byte load) or fp32 (two) row.
+struct Bf16x8 {
+  typedef uint16_t elem;
+  u32x4_t v;
+  __device__ __forceinline__ void load(const elem *p, bool ok = true) {  // zeros when not ok
+    v = ok ? *reinterpret_cast<const u32x4_t *>(p) : u32x4_t{0u, 0u, 0u, 0u};
+  }
+  __device__ __forceinline__ float operator[](int i) const {
+    return __uint_as_float(i & 1 ? v[i / 2] & 0xffff0000u : v[i / 2] << 16);
+  }
+};
+struct F32x8 {
+  typedef float elem;
+  f32x4_t v[2];
+  __device__ __forceinline__ void load(const elem *p, bool ok = true) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+      v[h] = ok ? reinterpret_cast<const f32x4_t *>(p)[h] : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  }
+  __device__ __forceinline__ float operator[](int i) const { return v[i / 4][i % 4]; }
+};
+
+// The same per-row quantisation for rows with K % 8 == 0, 16-byte aligned:
+// each thread holds up to VPT 8-element vectors of its row in registers
+// between the amax and the quantise pass and writes 8 bytes of qx at a time
+// (row-major, or in fragment order when FRAG).  Bit-identical to
 // dyn_quantize_kernel.
-template <int VPT, bool FRAG, bool ASYM>
-__global__ __launch_bounds__(256) void dyn_quantize_bf16_kernel(const uint16_t *x, int64_t K,
-                                                                 int8_t *qx, float *sx,
-                                                                 int32_t *azp, int32_t *zero,
-                                                                 int nzero) {
-  __shared__ float red[8];
+template <typename V, int NT, int VPT, bool FRAG, bool ASYM>
+__global__ __launch_bounds__(NT) void dyn_quantize_vec_kernel(const typename V::elem *x, int64_t K,
+                                                               int8_t *qx, float *sx, int32_t *azp,
+                                                               int32_t *zero, int nzero) {
+  __shared__ float red[NT / 32];
   const int tid = threadIdx.x;
   const int64_t m = blockIdx.x;
   zero_counters(zero, nzero, tid);
-  const u32x4_t *row = reinterpret_cast<const u32x4_t *>(x + m * K);
+  const typename V::elem *row = x + m * K;
   const int nv = (int)(K / 8);
-  u32x4_t v[VPT];
+  V v[VPT];
   float lo = 0.f, hi = 0.f;
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int j = tid + 256 * i;
-    v[i] = j < nv ? row[j] : u32x4_t{0u, 0u, 0u, 0u};
+    const int j = tid + NT * i;
+    v[i].load(row + 8 * j, j < nv);
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
-      const float e0 = __uint_as_float(v[i][w] << 16);
-      const float e1 = __uint_as_float(v[i][w] & 0xffff0000u);
+      const float e0 = v[i][2 * w], e1 = v[i][2 * w + 1];
       if (ASYM) {
         lo = fminf(lo, fminf(e0, e1));
         hi = fmaxf(hi, fmaxf(e0, e1));
@@ -168,7 +192,7 @@ __global__ __launch_bounds__(256) void dyn_quantize_bf16_kernel(const uint16_t *
       }
     }
   }
-  block_minmax(lo, hi, red, tid);
+  block_minmax<NT>(lo, hi, red, tid);
   float s, zp;
   row_qparams<ASYM>(lo, hi, s, zp);
   if (tid == 0) {
@@ -180,20 +204,79 @@ __global__ __launch_bounds__(256) void dyn_quantize_bf16_kernel(const uint16_t *
   u32x2_t *out = reinterpret_cast<u32x2_t *>(qx + m * K);
 #pragma unroll
   for (int i = 0; i < VPT; ++i) {
-    const int j = tid + 256 * i;
+    const int j = tid + NT * i;
     if (j >= nv) break;
     u32x2_t o;
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const uint32_t a0 = v[i][2 * h], a1 = v[i][2 * h + 1];
-      o[h] = q1(__uint_as_float(a0 << 16)) | (q1(__uint_as_float(a0 & 0xffff0000u)) << 8) |
-             (q1(__uint_as_float(a1 << 16)) << 16) | (q1(__uint_as_float(a1 & 0xffff0000u)) << 24);
-    }
+    for (int h = 0; h < 2; ++h)
+      o[h] = q1(v[i][4 * h]) | (q1(v[i][4 * h + 1]) << 8) | (q1(v[i][4 * h + 2]) << 16) |
+             (q1(v[i][4 * h + 3]) << 24);
     if (FRAG)
       *reinterpret_cast<u32x2_t *>(qx + qx_frag_offset(m, 8 * (int64_t)j, K)) = o;
     else
       out[j] = o;
   }
+}
+
+// Static quantisation of one value to the byte stored in qx (see
+// static_quantize_kernel).
+__device__ __forceinline__ int static_quant_one(float v, float inv, bool u8, float z) {
+  const float r = rintf(v * inv);
+  return u8 ? (int)fminf(fmaxf(r + z, 0.f), 255.f) - 128 : (int)fminf(fmaxf(r, -128.f), 127.f);
+}
+
+// static_quantize_kernel for K % 16 == 0 and 16-byte aligned x: 16 elements
+// per thread over the whole tensor, 16-byte loads and stores (the fragment
+// order keeps blocks of 16 whole).  3000 x 1024 bf16 and 3000 x 4096 u8: 11.7 us
+// each element by element.
+__global__ __launch_bounds__(256) void static_quantize_vec_kernel(
+    const void *x, int x_dt, int64_t M, int64_t K, int8_t *qx, int frag, const float *scale,
+    const int32_t *zp, float *sx, int32_t *azp, int32_t *zero, int nzero) {
+  zero_counters(zero, nzero, threadIdx.x);
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const float s = *scale;
+  const int32_t z = zp ? *zp : 0;
+  const bool u8 = x_dt == ZT_DT_U8 || ((x_dt == ZT_DT_F32 || x_dt == ZT_DT_BF16) && zp);
+  if (i < M) {
+    sx[i] = s;
+    if (azp) azp[i] = u8 ? z - 128 : z;
+  }
+  const int64_t per_row = K / 16;
+  if (i >= M * per_row) return;
+  const int64_t m = i / per_row, k = (i - m * per_row) * 16, at = i * 16;
+  u32x4_t o;
+  if (x_dt == ZT_DT_S8 || x_dt == ZT_DT_U8) {
+    o = *reinterpret_cast<const u32x4_t *>(static_cast<const int8_t *>(x) + at);
+    if (x_dt == ZT_DT_U8)
+#pragma unroll
+      for (int w = 0; w < 4; ++w) o[w] ^= 0x80808080u;  // x - 128 as s8
+  } else {
+    const float inv = __fdiv_rn(1.0f, s), zf = (float)z;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      float e[8];
+      if (x_dt == ZT_DT_BF16) {
+        Bf16x8 v;
+        v.load(static_cast<const uint16_t *>(x) + at + 8 * h);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = v[j];
+      } else {
+        F32x8 v;
+        v.load(static_cast<const float *>(x) + at + 8 * h);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = v[j];
+      }
+#pragma unroll
+      for (int w = 0; w < 2; ++w) {
+        uint32_t b = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          b |= ((uint32_t)static_quant_one(e[4 * w + j], inv, u8, zf) & 0xffu) << (8 * j);
+        o[2 * h + w] = b;
+      }
+    }
+  }
+  *reinterpret_cast<u32x4_t *>(qx + (frag ? qx_frag_offset(m, k, K) : at)) = o;
 }
 
 // Static per-tensor quantisation of zentorch_qlinear's activations, one
@@ -223,9 +306,7 @@ __global__ __launch_bounds__(256) void static_quantize_kernel(
     } else if (x_dt == ZT_DT_U8) {
       q = (int)reinterpret_cast<const uint8_t *>(x)[base + k] - 128;
     } else {
-      const float r = rintf(load_elem(x, x_dt, base + k) * inv);
-      q = u8 ? (int)fminf(fmaxf(r + (float)z, 0.f), 255.f) - 128
-             : (int)fminf(fmaxf(r, -128.f), 127.f);
+      q = static_quant_one(load_elem(x, x_dt, base + k), inv, u8, (float)z);
     }
     qx[frag ? qx_frag_offset(m, k, K) : base + k] = (int8_t)q;
   }
@@ -492,15 +573,19 @@ __device__ __forceinline__ void s8_tile_epilogue(const DynArgs &a, const int32_t
         const i32x4_t v = *reinterpret_cast<const i32x4_t *>(rows + row * AP + c4);
         float f[4];
         qs.scale(qs.correct(v, a.azp ? a.azp[min(m0 + row, M - 1)] : 0), sx_l[row], f);
-        *reinterpret_cast<f32x4_t *>(frows + row * AP + c4) = f32x4_t{f[0], f[1], f[2], f[3]};
+        if (!at_most_relu(a.post))
+          *reinterpret_cast<f32x4_t *>(frows + row * AP + c4) = f32x4_t{f[0], f[1], f[2], f[3]};
+        else if (m0 + row < M)
+          store_y4(a, qs, m0 + row, n, N, f, a.post.count != 0);
       }
+      if (at_most_relu(a.post)) return;
       post_ops_slab<T, RP>(frows, AP, c4, r0, a.post, m0, n, M, N);
 #pragma unroll 4
       for (int t = 0; t < T; ++t) {
         const int row = t * RP + r0;
         const f32x4_t v = *reinterpret_cast<const f32x4_t *>(frows + row * AP + c4);
-        const float f[4] = {v[0], v[1], v[2], v[3]};
-        if (m0 + row < M) store_y4(a, qs, m0 + row, n, N, f);
+        float f[4] = {v[0], v[1], v[2], v[3]};
+        if (m0 + row < M) store_y4(a, qs, m0 + row, n, N, f, false);
       }
       return;
     }
@@ -2106,27 +2191,42 @@ hipError_t launch_dyn_quantize(const void *x, int x_dt, int64_t M, int64_t K,
                                int32_t *azp, int32_t *zero, int nzero) {
   if (M == 0) return hipSuccess;
   if (frag && K % 64 != 0) return hipErrorInvalidValue;
-  const bool vec = x_dt == ZT_DT_BF16 && K % 8 == 0 &&
+  const bool vec = K % 8 == 0 &&
                    ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(qx)) & 15u) == 0;
   const int64_t per = (K / 8 + 255) / 256;  // 8-element vectors per thread
   const dim3 grid((unsigned)M), block(256);
   // up to 16 vectors per thread (K <= 32768); longer rows take the
   // element-wise kernel (measured: at K = 28672 the element-wise kernel made
-  // the op at M = 3..5, N = 8192 take 113-114 us)
+  // the op at M = 3..5, N = 8192 take 113-114 us; in fp32, 1000 x 1024 took
+  // 5.8 us there)
   if (vec && per <= 16) {
-    const uint16_t *xb = static_cast<const uint16_t *>(x);
-#define ZT_QB(V_)                                                                          \
-  if (per <= V_) {                                                                         \
-    if (azp)                                                                               \
-      frag ? dyn_quantize_bf16_kernel<V_, true, true><<<grid, block, 0, s>>>(xb, K, qx, sx, azp, zero, nzero) \
-           : dyn_quantize_bf16_kernel<V_, false, true><<<grid, block, 0, s>>>(xb, K, qx, sx, azp, zero, nzero); \
-    else                                                                                   \
-      frag ? dyn_quantize_bf16_kernel<V_, true, false><<<grid, block, 0, s>>>(xb, K, qx, sx, azp, zero, nzero) \
-           : dyn_quantize_bf16_kernel<V_, false, false><<<grid, block, 0, s>>>(xb, K, qx, sx, azp, zero, nzero); \
+#define ZT_QT(T_, NT_, V_, FRAG_, ASYM_)                                                   \
+  dyn_quantize_vec_kernel<T_, NT_, V_, FRAG_, ASYM_><<<grid, dim3(NT_), 0, s>>>(           \
+      static_cast<const T_::elem *>(x), K, qx, sx, azp, zero, nzero)
+#define ZT_QV(T_, NT_, V_)                                                                 \
+  if (K / 8 <= NT_ * V_) {                                                                 \
+    if (azp) {                                                                             \
+      if (frag) ZT_QT(T_, NT_, V_, true, true);                                            \
+      else ZT_QT(T_, NT_, V_, false, true);                                                \
+    } else {                                                                               \
+      if (frag) ZT_QT(T_, NT_, V_, true, false);                                           \
+      else ZT_QT(T_, NT_, V_, false, false);                                               \
+    }                                                                                      \
     return hipGetLastError();                                                              \
   }
-    ZT_QB(2) ZT_QB(4) ZT_QB(8) ZT_QB(16)
-#undef ZT_QB
+    // Few rows: their workgroups do not fill the GPU, so a row's time is one
+    // thread's, and longer rows take more threads (8 x 14336: 5.8 us with 256)
+    const bool few = M <= 256 && per > 2;
+    if (x_dt == ZT_DT_BF16) {
+      if (few) { ZT_QV(Bf16x8, 1024, 1) ZT_QV(Bf16x8, 1024, 2) ZT_QV(Bf16x8, 1024, 4) }
+      ZT_QV(Bf16x8, 256, 2) ZT_QV(Bf16x8, 256, 4) ZT_QV(Bf16x8, 256, 8) ZT_QV(Bf16x8, 256, 16)
+    } else {
+      if (few) { ZT_QV(F32x8, 1024, 1) ZT_QV(F32x8, 1024, 2) ZT_QV(F32x8, 1024, 4) }
+      ZT_QV(F32x8, 256, 1) ZT_QV(F32x8, 256, 2) ZT_QV(F32x8, 256, 4) ZT_QV(F32x8, 256, 8)
+      ZT_QV(F32x8, 256, 16)
+    }
+#undef ZT_QV
+#undef ZT_QT
   }
   if (azp)
     dyn_quantize_kernel<true><<<grid, block, 0, s>>>(x, x_dt, K, qx, sx, (int)frag, azp,
@@ -2142,6 +2242,12 @@ hipError_t launch_static_quantize(const void *x, int x_dt, int64_t M, int64_t K,
                                   int32_t *azp, hipStream_t s, int32_t *zero, int nzero) {
   if (M == 0) return hipSuccess;
   if (frag && K % 64 != 0) return hipErrorInvalidValue;
+  if (K % 16 == 0 &&
+      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(qx)) & 15u) == 0) {
+    static_quantize_vec_kernel<<<dim3((unsigned)((M * (K / 16) + 255) / 256)), dim3(256), 0, s>>>(
+        x, x_dt, M, K, qx, (int)frag, scale, zp, sx, azp, zero, nzero);
+    return hipGetLastError();
+  }
   static_quantize_kernel<<<dim3((unsigned)M), dim3(256), 0, s>>>(x, x_dt, K, qx, (int)frag, scale,
                                                                  zp, sx, azp, zero, nzero);
   return hipGetLastError();

@@ -41,6 +41,12 @@ struct QuadScales {
   }
 };
 
+// Whether the post-ops are at most one relu, which costs one instruction on
+// the way to the store and no pass of its own.
+__device__ __forceinline__ bool at_most_relu(const PostOps &p) {
+  return p.count == 0 || (p.count == 1 && p.ids[0] == ZT_PO_RELU);
+}
+
 // Columns n..n+3 of row m of the raw sums / of y.
 __device__ __forceinline__ void store_sums4(const DynArgs &a, int m, int n, int N, i32x4_t v) {
   int32_t *dst = reinterpret_cast<int32_t *>(a.y) + (int64_t)m * N + n;
@@ -54,7 +60,10 @@ __device__ __forceinline__ void store_sums4(const DynArgs &a, int m, int n, int 
 }
 
 __device__ __forceinline__ void store_y4(const DynArgs &a, const QuadScales &q, int m, int n, int N,
-                                         const float (&f)[4]) {
+                                         float (&f)[4], bool relu) {
+  if (relu)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) f[r] = unary_op(ZT_PO_RELU, f[r]);
   if (a.y_dt != ZT_DT_U8 && a.y_dt != ZT_DT_S8) {
     store4(a.y, a.y_dt, N, m, n, N, f);
     return;

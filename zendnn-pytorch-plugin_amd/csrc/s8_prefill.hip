@@ -191,13 +191,13 @@ void s8_prefill_kernel(DynArgs a, int tiles_m, int tiles_n, int group_m) {
         const i32x4_t v = sums(t);
         if (m < M && n < N) store_sums4(a, m, n, N, qs.correct(v, azp_l[i * 32 + row]));
       }
-    } else if (!a.post.count) {
+    } else if (at_most_relu(a.post)) {
 #pragma unroll 4
       for (int t = 0; t < 8; ++t) {
         const int row = t * 4 + r0, m = mb + row;
         float f[4];
         qs.scale(qs.correct(sums(t), azp_l[i * 32 + row]), sx_l[i * 32 + row], f);
-        if (m < M && n < N) store_y4(a, qs, m, n, N, f);
+        if (m < M && n < N) store_y4(a, qs, m, n, N, f, a.post.count != 0);
       }
     } else {
 #pragma unroll 4
@@ -212,8 +212,8 @@ void s8_prefill_kernel(DynArgs a, int tiles_m, int tiles_n, int group_m) {
       for (int t = 0; t < 8; ++t) {
         const int row = t * 4 + r0, m = mb + row;
         const f32x4_t v = *reinterpret_cast<const f32x4_t *>(fslab + row * SP + c4);
-        const float f[4] = {v[0], v[1], v[2], v[3]};
-        if (m < M && n < N) store_y4(a, qs, m, n, N, f);
+        float f[4] = {v[0], v[1], v[2], v[3]};
+        if (m < M && n < N) store_y4(a, qs, m, n, N, f, false);
       }
     }
     __builtin_amdgcn_wave_barrier();
