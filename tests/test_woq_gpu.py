@@ -751,3 +751,44 @@ def test_zero_points_17_to_64_rows(M, K, N, knobs, capfd):
     capfd.readouterr()
     run_case(M, K, N, K // 128, zp="int", seed=M + N, bias=True)
     assert "woq prefill" in capfd.readouterr().err
+
+
+# 8-bit zero points and groups of 32 / 64 on the decode kernels: the stream
+# kernel (x whole, in K phases, several token tiles), the wide kernel (both
+# token tiles, padded and uneven splits), the merged gate_up on both; ragged N
+def group_case(M, K, N, gs, zp, seed):
+    x, q, wp, s, z, b = make_case(M, K, N, K // gs, seed, zp="int" if zp else None, bias=True)
+    return x, wp, s, z.to(zp) if zp else None, b
+
+
+@pytest.mark.parametrize("M,K,N,kernel", [
+    (1, 1024, 40, "stream"), (4, 3584, 132, "stream"), (16, 4096, 260, "stream"),
+    (9, 14336, 68, "stream"), (3, 2176, 36, "stream"), (30, 4096, 260, "stream"),
+    (64, 2048, 132, "stream"), (17, 11008, 1540, "wide"), (33, 3584, 4164, "wide"),
+    (64, 1280, 4164, "wide"), (12, 13824, 5124, "wide"), (17, 11008, 136, "prefill")])
+@pytest.mark.parametrize("gs,zp", [(128, torch.int8), (64, torch.uint8), (64, None),
+                                   (32, torch.int8), (32, None), (256, torch.uint8)])
+def test_group_modes_decode(M, K, N, kernel, gs, zp, knobs, capfd):
+    if K % gs or (K // gs * gs != K):
+        pytest.skip("K is not whole groups")
+    knobs.set("ZT_WOQ_DEBUG", "1")
+    x, wp, s, z, b = group_case(M, K, N, gs, zp, M + K + N + gs)
+    y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b, post_ops=("relu",))
+    xd, wd, sd, zd, bd = gpu(x, wp, s, z, b)
+    capfd.readouterr()
+    y = C.woq_linear(xd, wd, sd, zd, bd, post_ops=("relu",))
+    assert f"woq {kernel}" in capfd.readouterr().err
+    check_close(y, y_ref)
+
+
+@pytest.mark.parametrize("M,K,I", [(1, 1024, 48), (5, 4096, 64), (16, 2048, 160), (20, 1024, 64),
+                                   (64, 4096, 8256)])
+@pytest.mark.parametrize("gs,zp", [(128, torch.int8), (64, None), (32, torch.uint8)])
+def test_group_modes_gate_up(M, K, I, gs, zp):
+    x, wp, s, z, b = group_case(M, K, 2 * I, gs, zp, M + K + I)
+    half = lambda t, lo: None if t is None else (t[lo:lo + I] if t.dim() == 1 else
+                                                 t[:, lo:lo + I].contiguous())
+    up = O.woq_linear(x, wp[I:].contiguous(), half(s, I), zero_points=half(z, I), bias=half(b, I))
+    y_ref = O.woq_linear(x, wp[:I].contiguous(), half(s, 0), zero_points=half(z, 0),
+                         bias=half(b, 0), post_ops=("silu", "mul"), post_bufs=[up])
+    check_close(C.woq_linear_gate_up(*gpu(x, wp, s, z, b)), y_ref)

@@ -279,10 +279,10 @@ size_t zt_woq_linear_workspace_size(int64_t M, int64_t K, int64_t N,
   a.x = reinterpret_cast<const void *>(256);
   a.w = reinterpret_cast<const uint32_t *>(256);
   // the prefill GEMM's K-split partials (few tiles)
-  const size_t gemm = zt::woq_gemm_workspace(M, N, K);
-  if (M > kWoqRowBlock || zt::woq_select_kernel(a) != zt::kWoqDecode) return std::max(wide, gemm);
   zt::DecodePlan p;
-  if (!zt::woq_decode_plan(M, N, K, &p)) return std::max(wide, gemm);
+  if (M > kWoqRowBlock || zt::woq_select_kernel(a) != zt::kWoqDecode ||
+      !zt::woq_decode_plan(M, N, K, &p))
+    return std::max(wide, zt::woq_gemm_workspace(M, N, K));
   return std::max(wide, zt::woq_decode_workspace(p, M, N));
 }
 
@@ -339,15 +339,24 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   zt::WidePlan wp;
-  if (zt::woq_wide_ok(a, &wp)) {
-    const size_t need = zt::woq_wide_workspace(wp, M, N);
-    if (need && (!workspace || workspace_bytes < need))
+  const bool wide = zt::woq_wide_ok(a, &wp);
+  const size_t need = wide ? zt::woq_wide_workspace(wp, M, N) : 0;
+  const bool room = !need || (workspace && workspace_bytes >= need);
+  // (zero points and groups of 32 / 64 have other kernels to go to without it)
+  if (wide && (room || (!zp && (G == 1 || (K / G) % 128 == 0)))) {
+    if (!room)
       return fail(ZT_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op, need,
                   workspace ? workspace_bytes : (size_t)0);
     return hip_status(zt::launch_woq_wide(a, wp, workspace, s), op);
   }
-  // 17..64 rows with zero points or fp32 scales, which the wide kernel does
-  // not take: the prefill GEMM, K split over the workspace, reads the weights
+  {
+    const char *f = zt::knob(zt::kKnobWoqForceKernel);
+    hipError_t err = hipSuccess;
+    if ((!f || !std::strcmp(f, "decode")) && zt::woq_try_group_stream(a, s, &err))
+      return hip_status(err, op);
+  }
+  // 17..64 rows with fp32 scales or zero points the wide kernel does not
+  // take: the prefill GEMM, K split over the workspace, reads the weights
   // once where the decode kernels' general modes pay their longer
   // dequantisation per row block (zero points, 24 / 64 rows: 4096 x 4096 17.8 /
   // 34.6 -> 16.8 / 21.2 us, 18944 x 3584 68.7 / 167 -> 31.0 / 35.1,
@@ -418,8 +427,15 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   hipError_t err = hipSuccess;
   if (zt::woq_try_stream_gate_up(a, s, &err)) return hip_status(err, op);
   if (zt::woq_try_wide_gate_up(a, s, &err)) return hip_status(err, op);
+  // the prefill kernel's merged form past 64 rows, and where the plain linear
+  // would take that kernel too; the decode kernels keep the two steps
   const char *forced = zt::knob(zt::kKnobWoqGemm);
-  if ((!forced || forced[0] == 'p') && zt::woq_prefill_ok(a))
+  zt::WidePlan wp;
+  const bool decode = M <= kWoqRowBlockMax && !(forced && forced[0] == 'p') &&
+                      (zt::woq_wide_ok(a, &wp) || zt::woq_group_stream_ok(a) ||
+                       (M > kWoqRowBlock ? !zp && scales_dtype != ZT_DT_F32 && woq_use_row_blocks(a)
+                                         : zt::woq_select_kernel(a) == zt::kWoqDecode));
+  if (!decode && (!forced || forced[0] == 'p') && zt::woq_prefill_ok(a))
     return hip_status(zt::launch_woq_prefill(a, true, nullptr, 0, s), op);
   // two steps: the full [M, N] linear in fp32 into the workspace, then
   // silu(gate) * up over its halves

@@ -121,9 +121,17 @@ __global__ __launch_bounds__(256) void woq_generic_kernel(WoqArgs a) {
 // ------------------------------------------------------------- decode
 constexpr unsigned kCounterSlots = 1024;  // 4096-byte counter region
 
-// Dequantisation modes of the decode kernel: signed int4 with bf16 scales
-// (the fast path), or the general path with bf16 / fp32 scales.
-enum DecodeMode { kDecFast = 0, kDecGenBf16 = 1, kDecGenF32 = 2 };
+// Dequantisation modes of the decode kernels: signed int4 with bf16 scales
+// in groups of 128 and up (the fast path); the general path with bf16 / fp32
+// scales; and, on the stream and wide kernels, bf16 scales in groups of 32
+// and up (a lane of the decode layout holds exactly one block of 32), signed
+// or with 8-bit zero points, at the fast path's one FMA per weight.
+enum DecodeMode { kDecFast = 0, kDecGenBf16 = 1, kDecGenF32 = 2, kDecS4G = 3, kDecU4G = 4 };
+
+// Modes whose scales (and zero points) the stream kernel stages in LDS.
+__host__ __device__ constexpr bool dec_staged(int mode) {
+  return mode == kDecFast || mode == kDecS4G || mode == kDecU4G;
+}
 
 template <int MODE>
 __device__ __forceinline__ float scale_at(const WoqArgs &a, int64_t i) {
@@ -134,8 +142,10 @@ __device__ __forceinline__ float scale_at(const WoqArgs &a, int64_t i) {
 template <int MODE>
 __device__ __forceinline__ bf16x8_t dq_word(uint32_t w, float s, float z, int zmode) {
   u32x4_t v;
-  if (MODE == kDecFast)
+  if (MODE == kDecFast || MODE == kDecS4G)
     v = dq8_s4_bf16scale(w, s, s * 0.0625f, -1032.f * s, -72.f * s);
+  else if (MODE == kDecU4G)
+    v = dq8_u4_bf16scale(w, s, z);
   else
     v = dq8_general(w, dq_general_params(zmode, s, z));
   return __builtin_bit_cast(bf16x8_t, v);
@@ -419,6 +429,14 @@ __host__ __device__ inline int stream_phase_pitch(int kp) { return (kp + 511) / 
 __host__ __device__ constexpr size_t stream_scale_bytes(int G, int tpw) {
   return (size_t)((G * tpw + 7) / 8) * 256;
 }
+// kDecU4G: their zero points behind them, [G][TPW*16] bytes
+__host__ __device__ constexpr size_t stream_zp_bytes(int G, int tpw) {
+  return (size_t)((G * tpw + 15) / 16) * 256;
+}
+__host__ __device__ constexpr size_t stream_staged_bytes(int mode, int G, int tpw) {
+  return (dec_staged(mode) ? stream_scale_bytes(G, tpw) : 0) +
+         (mode == kDecU4G ? stream_zp_bytes(G, tpw) : 0);
+}
 
 // gu > 0 (merged gate_up, fast mode, TPW even, P == MT == 1): weight rows
 // [0, gu) are the gate and [gu, 2 gu) the up projection; tile 2i of the
@@ -441,6 +459,7 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
     return gu ? (t & 1) * gu + (blockIdx.x * (TPW / 2) + (t >> 1)) * 16 : (t0 + t) * 16;
   };
   const int zmode = zp_mode_of(a.zp, a.zp_dt);
+  const int zsx = a.zp_dt == ZT_DT_S8 ? 0x80 : 0;  // sign bit of the staged zero points
   const int s_bytes = MODE == kDecGenF32 ? 4 : 2;
   const auto w_rsrc = make_rsrc(a.w, (uint32_t)((int64_t)N * KW * 4));
   const auto s_rsrc = make_rsrc(a.scales, (uint32_t)(a.G * N * s_bytes));
@@ -485,7 +504,20 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
   // so the wait for x below covers them too.
   const uint16_t *sl = reinterpret_cast<const uint16_t *>(
       smem + stream_scale_offset(stream_slab_bytes(NW, TPW, MT), (size_t)M * XP * 2));
-  if (MODE == kDecFast) {
+  const uint8_t *zl =
+      reinterpret_cast<const uint8_t *>(sl) + stream_scale_bytes((int)a.G, TPW);
+  if (MODE == kDecU4G) {
+    // one DMA instruction moves the zero points of 16/TPW groups (N % 4 == 0)
+    const int G = (int)a.G, gbytes = TPW * 16;
+    const auto z_rsrc = make_rsrc(a.zp, (uint32_t)(a.G * N));
+    for (int i = wv; i < (G * TPW + 15) / 16; i += NW) {
+      const int byte = i * 256 + lane * 4, g = byte / gbytes, b = byte - g * gbytes;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          z_rsrc, (lds_ptr_t)(zl + i * 256), 4,
+          g < G ? (uint32_t)(g * N + rowbase(b >> 4) + (b & 15)) : kOobOffset, 0, 0, 0);
+    }
+  }
+  if (dec_staged(MODE)) {
     const int G = (int)a.G, gbytes = TPW * 32;
     const int ns = (G * TPW + 7) / 8;
     for (int i = wv; i < ns; i += NW) {
@@ -517,7 +549,7 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
         sr[t][c] = __builtin_amdgcn_raw_buffer_load_b32(s_rsrc, sidx * 4u, 0, 0);
       else if (MODE == kDecGenBf16)
         sr[t][c] = __builtin_amdgcn_raw_buffer_load_b16(s_rsrc, sidx * 2u, 0, 0);
-      zr[t][c] = (MODE != kDecFast && zmode) ? load_elem(a.zp, a.zp_dt, sidx) : 0.f;
+      zr[t][c] = (!dec_staged(MODE) && zmode) ? load_elem(a.zp, a.zp_dt, sidx) : 0.f;
     }
   };
   // the first D chunks now, chunk c + D when chunk c is computed
@@ -541,7 +573,7 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
           *reinterpret_cast<const u32x4_t *>(xp + (int64_t)m * a.ldx + k8 * 8);
     }
   }
-  if (P == 1 && MODE == kDecFast && x_dma) {
+  if (P == 1 && dec_staged(MODE) && x_dma) {
     constexpr int after = TPW * D > 63 ? 63 : TPW * D;
     __builtin_amdgcn_s_waitcnt((after & 15) | ((after >> 4) << 14) | (7 << 4) | (15 << 8));
     asm volatile("s_barrier" ::: "memory");
@@ -571,13 +603,16 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
       bf16x8_t wb[TPW][4];
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
-        const uint32_t sb =
-            MODE == kDecFast
-                ? (uint32_t)sl[((min(kc, C - 1) >> cpg_shift) & gmask) * (TPW * 16) + t * 16 + lr]
-                : sr[t][c];
+        // the lane's scale group: cpg_shift counts chunks in the fast mode,
+        // the lane's blocks of 32 in the group modes
+        const int at = (MODE == kDecFast ? ((min(kc, C - 1) >> cpg_shift) & gmask)
+                                         : (((min(kc, C - 1) * 4 + lg) >> cpg_shift) & gmask)) *
+                           (TPW * 16) + t * 16 + lr;
+        const uint32_t sb = dec_staged(MODE) ? (uint32_t)sl[at] : sr[t][c];
         const float sc = MODE == kDecGenF32 ? __uint_as_float(sb) : __uint_as_float(sb << 16);
+        const float zc = MODE == kDecU4G ? (float)(((int)zl[at] ^ zsx) - zsx) : zr[t][c];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wb[t][i] = dq_word<MODE>(wr[t][c][i], sc, zr[t][c], zmode);
+        for (int i = 0; i < 4; ++i) wb[t][i] = dq_word<MODE>(wr[t][c][i], sc, zc, zmode);
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
@@ -1991,17 +2026,30 @@ static hipError_t launch_stream_t(const WoqArgs &a, hipStream_t s, int shift, in
       stream_scale_offset(stream_slab_bytes(NW, TPW, MT),
                           (size_t)a.M *
                               (P == 1 ? stream_x_pitch((int)a.K) : stream_phase_pitch((int)(a.K / P))) * 2) +
-      (mode == kDecFast ? stream_scale_bytes((int)a.G, TPW) : 0);
+      stream_staged_bytes(mode, (int)a.G, TPW);
   dim3 grid((unsigned)((tiles + TPW - 1) / TPW)), block(64 * NW);
-  if (mode == kDecFast)
+  if (mode == kDecFast) {
     woq_stream_kernel<NW, CPW, TPW, kDecFast, P, MT><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
-  else if (P > 1 || MT > 1)
-    return hipErrorInvalidValue;  // phases and token tiles are built for the fast mode only
-  else if (mode == kDecGenBf16)
-    woq_stream_kernel<NW, CPW, TPW, kDecGenBf16, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
-  else
-    woq_stream_kernel<NW, CPW, TPW, kDecGenF32, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
-  return hipGetLastError();
+    return hipGetLastError();
+  }
+  if (mode == kDecS4G || mode == kDecU4G) {
+    if constexpr (NW == 8) {
+      if (mode == kDecS4G)
+        woq_stream_kernel<NW, CPW, TPW, kDecS4G, P, MT><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
+      else
+        woq_stream_kernel<NW, CPW, TPW, kDecU4G, P, MT><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
+      return hipGetLastError();
+    }
+    return hipErrorInvalidValue;
+  }
+  if constexpr (P == 1 && MT == 1) {
+    if (mode == kDecGenBf16)
+      woq_stream_kernel<NW, CPW, TPW, kDecGenBf16, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
+    else
+      woq_stream_kernel<NW, CPW, TPW, kDecGenF32, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
+    return hipGetLastError();
+  }
+  return hipErrorInvalidValue;  // phases and token tiles are built for the staged modes only
 }
 
 // ------------------------------------------------------ lean decode
@@ -2293,7 +2341,7 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
     return stream_scale_offset(stream_slab_bytes(nw, tpw, mt),
                                (size_t)a.M *
                                    (p == 1 ? stream_x_pitch((int)a.K) : stream_phase_pitch((int)(a.K / p))) * 2) +
-               (mode == kDecFast ? stream_scale_bytes((int)a.G, tpw) : 0) <=
+               stream_staged_bytes(mode, (int)a.G, tpw) <=
            kStreamLdsMax;
   };
   // x whole would leave room for one workgroup per CU while the grid makes
@@ -2302,12 +2350,12 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
   // 20.4 / 21.3 us with x whole on 320 workgroups of two tiles)
   const int tpw0 = tpw;
   const bool prefer_phases =
-      !e && mt == 1 && mode == kDecFast && a.x_dt == ZT_DT_BF16 && fits(1) &&
+      !e && mt == 1 && dec_staged(mode) && a.x_dt == ZT_DT_BF16 && fits(1) &&
       (size_t)a.M * stream_x_pitch((int)a.K) * 2 > kStreamLdsMax / 2 && (tiles + tpw - 1) / tpw > 256;
   if (mt > 1 || !fits(1) || prefer_phases) {
     // several token tiles or K phases: 8 waves, one tile each, fast mode,
     // the fewest phases whose x range fits
-    if (e || mode != kDecFast || a.x_dt != ZT_DT_BF16) return false;
+    if (e || !dec_staged(mode) || a.x_dt != ZT_DT_BF16) return false;
     nw = 8, tpw = 1;
     for (int p : {1, 2, 4, 8}) {
       const int cp = C / p;
@@ -2430,22 +2478,25 @@ constexpr size_t woq_wide_xstage() {
   return (size_t)(32 * MT) * (kWideKP * 2);
 }
 
-template <int MT>
+// SPC: scale groups per 128-k chunk (1: groups of 128 and up)
+template <int MT, int SPC, bool ZP>
 constexpr size_t woq_wide_lds() {
-  // x stages, scale stages [round][2 chunks][128 rows], and a spare 256-byte
-  // block the out-of-range scale DMA of waves 2..7 writes
-  const size_t x = kWideRound * woq_wide_xstage<MT>() + kWideRound * 2 * (kWideRows * 2) + 256;
+  // x stages, scale stages [round][2 chunks][SPC][128 rows], with ZP the
+  // zero-point stages (128 bytes of 256 each), and a spare 256-byte block the
+  // out-of-range DMA of the other waves writes
+  const size_t x = kWideRound * woq_wide_xstage<MT>() +
+                   kWideRound * 2 * SPC * (kWideRows * 2) * (ZP ? 2 : 1) + 256;
   const size_t tile = (size_t)(32 * MT) * (kWideRows + 4) * 4;
   return x > tile ? x : tile;
 }
 
-template <int MT, bool PAD>
+template <int MT, bool PAD, int SPC, bool ZP>
 __global__ __launch_bounds__(512) void woq_wide_kernel(WoqArgs a, int pps, int cpg_shift, int gmask,
                                                        float *partial, int gu) {
   extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
   constexpr int XS = (int)woq_wide_xstage<MT>();
   constexpr int XL = 2 * MT;        // x DMA (two token rows each) per wave per phase
-  constexpr int OPS = 3 + XL;       // loads per wave per phase: 2 weight tiles, scales, x
+  constexpr int OPS = 3 + ZP + XL;  // loads per wave per phase: 2 weight tiles, scales, zp, x
   constexpr int WAIT = vmcnt_imm_woq((kWideAhead - 1) * OPS);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2476,14 +2527,21 @@ __global__ __launch_bounds__(512) void woq_wide_kernel(WoqArgs a, int pps, int c
 
   u32x4_t wq[kWideRound][2];
   unsigned char *sbuf0 = smem + kWideRound * XS;
+  constexpr int SLOTS = kWideRound * 2 * SPC;  // 256-byte scale rows in LDS
+  unsigned char *zbuf0 = sbuf0 + SLOTS * (kWideRows * 2);
+  unsigned char *spare = zbuf0 + (ZP ? SLOTS * (kWideRows * 2) : 0);
+  const auto z_rs = make_rsrc(a.zp, ZP ? (uint32_t)(a.G * N) : 0u);
+  const int zsx = a.zp_dt == ZT_DT_S8 ? 0x80 : 0;  // the zero points' sign bit
   // Load i of phase ph.  The out-of-range bit is ORed into the offsets
   // (valid offsets stay below it): a select on the wave-uniform condition
   // would be compiled into branches around each load.
   //  0, 1: the weight tiles of the lane's low / high row (register set `set`)
-  //  2:    the scales: waves 0 and 1 move chunk wv's 128 row scales (one
-  //        256-byte DMA; N % 4 == 0 keeps the dwords aligned), the others an
-  //        out-of-range DMA into the spare block, so no branch surrounds it
-  //  3..:  x token rows 2 (wv + 8 i) and 2 (wv + 8 i) + 1, 512 bytes each
+  //  2:    the scales: waves 0 .. 2 SPC - 1 move the 128 row scales of group
+  //        wv of the phase's 2 SPC (one 256-byte DMA; N % 4 == 0 keeps the
+  //        dwords aligned), the others an out-of-range DMA into the spare
+  //        block, so no branch surrounds it
+  //  3:    with ZP their zero points likewise (lanes 0..31, four rows each)
+  //  then: x token rows 2 (wv + 8 i) and 2 (wv + 8 i) + 1, 512 bytes each
   auto load = [&](int i, int ph, int set) {
     const uint32_t oob = ph < pend ? 0u : kOobOffset;
     if (i < 2) {
@@ -2491,16 +2549,24 @@ __global__ __launch_bounds__(512) void woq_wide_kernel(WoqArgs a, int pps, int c
       const uint32_t off = i == 0 ? (off_lo + kc * 64u) | oob_lo : (off_hi + kc * 64u) | oob_hi;
       wq[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
           w_rs, off | oob, 0, 0));
-    } else if (i == 2) {
-      const int ch = wv & 1;
-      const uint32_t g = ((uint32_t)(ph * 2 + ch) >> cpg_shift) & (uint32_t)gmask;
-      const uint32_t soob = wv < 2 ? 0u : kOobOffset;
-      const int slot = wv < 2 ? (ph & (kWideRound - 1)) * 2 + ch : 2 * kWideRound;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          s_rs, (lds_ptr_t)(sbuf0 + slot * (kWideRows * 2)), 4,
-          ((g * (uint32_t)N + (uint32_t)row_of(2 * lane)) * 2u) | oob | soob, 0, 0, 0);
+    } else if (i == 2 || (ZP && i == 3)) {
+      const bool mine = wv < 2 * SPC;
+      const uint32_t kc = (uint32_t)(ph * 2 + (wv / SPC & 1));
+      const uint32_t g = SPC == 1 ? (kc >> cpg_shift) & (uint32_t)gmask
+                                  : kc * SPC + (uint32_t)(wv % SPC);
+      const uint32_t soob = mine ? 0u : kOobOffset;
+      const int slot = ((ph & (kWideRound - 1)) * 2 * SPC + wv) * (kWideRows * 2);
+      if (i == 2)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            s_rs, (lds_ptr_t)(mine ? sbuf0 + slot : spare), 4,
+            ((g * (uint32_t)N + (uint32_t)row_of(2 * lane)) * 2u) | oob | soob, 0, 0, 0);
+      else
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(
+            z_rs, (lds_ptr_t)(mine ? zbuf0 + slot : spare), 4,
+            (g * (uint32_t)N + (uint32_t)row_of(4 * (lane & 31))) | oob | soob |
+                (lane < 32 ? 0u : kOobOffset), 0, 0, 0);
     } else {
-      const int r = 2 * (wv + 8 * (i - 3));
+      const int r = 2 * (wv + 8 * (i - 3 - ZP));
       const int t = r + hl;
       const int c = l32 ^ (t & 15);
       const uint32_t off = (uint32_t)(t * ldx2 + ph * (kWideKP * 2) + c * 16) |
@@ -2530,10 +2596,16 @@ __global__ __launch_bounds__(512) void woq_wide_kernel(WoqArgs a, int pps, int c
         const int cc = kh * 16 + 8 * hl + q;
         xf[q][j] = *reinterpret_cast<const bf16x8_t *>(buf + t * (kWideKP * 2) + ((cc ^ (t & 15)) * 16));
       }
-    const float sc = __uint_as_float(
-        (uint32_t)reinterpret_cast<const uint16_t *>(
-            sbuf0 + ((ph & (kWideRound - 1)) * 2 + kh) * (kWideRows * 2))[rw * 32 + l32]
-        << 16);
+    // a lane's blocks of 32: 2 hl (steps 0..3) and 2 hl + 1 of its chunk
+    float sc[2], zc[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int g = SPC == 1 ? 0 : SPC == 2 ? hl : 2 * hl + b;
+      const int slot = (((ph & (kWideRound - 1)) * 2 + kh) * SPC + g) * (kWideRows * 2);
+      sc[b] = __uint_as_float(
+          (uint32_t)reinterpret_cast<const uint16_t *>(sbuf0 + slot)[rw * 32 + l32] << 16);
+      zc[b] = ZP ? (float)(((int)zbuf0[slot + rw * 32 + l32] ^ zsx) - zsx) : 0.f;
+    }
     u32x4_t w0 = wq[set][0], w1 = wq[set][1];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2548,7 +2620,8 @@ __global__ __launch_bounds__(512) void woq_wide_kernel(WoqArgs a, int pps, int c
         load(2 + q, ph + kWideAhead, 0);
         __builtin_amdgcn_sched_barrier(kSchedAllButVmem);
       }
-      const bf16x8_t wb = dq_word<kDecFast>(q < 4 ? w0[q] : w1[q - 4], sc, 0.f, 0);
+      const bf16x8_t wb =
+          dq_word<ZP ? kDecU4G : kDecFast>(q < 4 ? w0[q] : w1[q - 4], sc[q / 4], zc[q / 4], 0);
 #pragma unroll
       for (int j = 0; j < MT; ++j)
         acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb, xf[q][j], acc[j], 0, 0, 0);
@@ -2722,16 +2795,31 @@ static hipError_t launch_splitk_reduce(const WoqArgs &a, const float *partial, i
   return hipGetLastError();
 }
 
-static void launch_wide_t(const WoqArgs &a, const WidePlan &p, dim3 grid, int shift, int gmask,
+template <int SPC, bool ZP>
+static void launch_wide_q(const WoqArgs &a, const WidePlan &p, dim3 grid, int shift, int gmask,
                           float *partial, int gu, hipStream_t s) {
   if (p.mt == 1 && !p.pad)
-    woq_wide_kernel<1, false><<<grid, dim3(512), woq_wide_lds<1>(), s>>>(a, p.pps, shift, gmask, partial, gu);
+    woq_wide_kernel<1, false, SPC, ZP><<<grid, dim3(512), woq_wide_lds<1, SPC, ZP>(), s>>>(a, p.pps, shift, gmask, partial, gu);
   else if (p.mt == 1)
-    woq_wide_kernel<1, true><<<grid, dim3(512), woq_wide_lds<1>(), s>>>(a, p.pps, shift, gmask, partial, gu);
+    woq_wide_kernel<1, true, SPC, ZP><<<grid, dim3(512), woq_wide_lds<1, SPC, ZP>(), s>>>(a, p.pps, shift, gmask, partial, gu);
   else if (!p.pad)
-    woq_wide_kernel<2, false><<<grid, dim3(512), woq_wide_lds<2>(), s>>>(a, p.pps, shift, gmask, partial, gu);
+    woq_wide_kernel<2, false, SPC, ZP><<<grid, dim3(512), woq_wide_lds<2, SPC, ZP>(), s>>>(a, p.pps, shift, gmask, partial, gu);
   else
-    woq_wide_kernel<2, true><<<grid, dim3(512), woq_wide_lds<2>(), s>>>(a, p.pps, shift, gmask, partial, gu);
+    woq_wide_kernel<2, true, SPC, ZP><<<grid, dim3(512), woq_wide_lds<2, SPC, ZP>(), s>>>(a, p.pps, shift, gmask, partial, gu);
+}
+
+static void launch_wide_t(const WoqArgs &a, const WidePlan &p, dim3 grid, int shift, int gmask,
+                          float *partial, int gu, hipStream_t s) {
+  const int64_t gs = a.G == 1 ? 128 : a.K / a.G;
+  if (gs == 32)
+    a.zp ? launch_wide_q<4, true>(a, p, grid, shift, gmask, partial, gu, s)
+         : launch_wide_q<4, false>(a, p, grid, shift, gmask, partial, gu, s);
+  else if (gs == 64)
+    a.zp ? launch_wide_q<2, true>(a, p, grid, shift, gmask, partial, gu, s)
+         : launch_wide_q<2, false>(a, p, grid, shift, gmask, partial, gu, s);
+  else
+    a.zp ? launch_wide_q<1, true>(a, p, grid, shift, gmask, partial, gu, s)
+         : launch_wide_q<1, false>(a, p, grid, shift, gmask, partial, gu, s);
 }
 
 // Whether the stream kernel takes a call of up to 16 rows of this shape
@@ -2784,7 +2872,7 @@ bool woq_wide_plan(int64_t M, int64_t N, int64_t K, int64_t G, WidePlan *p) {
   // 24.6 us there against 11.8 / 14.4 here)
   if (M <= 64 && N <= 4096 && N * K <= (int64_t)4096 * 4096 && !forced) return false;
   const int64_t gs = K / G, cpg = gs / 128;
-  if (G != 1 && (gs % 128 || (cpg & (cpg - 1)))) return false;
+  if (G != 1 && gs != 32 && gs != 64 && (gs % 128 || (cpg & (cpg - 1)))) return false;
   const int phases = (int)(K / kWideKP);
   const int64_t blocks = (N + kWideRows - 1) / kWideRows;
   // the most K splits (a divisor of the phase count) of whole rounds of
@@ -2835,8 +2923,11 @@ bool woq_wide_ok(const WoqArgs &a, WidePlan *p) {
   const char *f = knob(kKnobWoqForceKernel);  // another forced kernel skips this one
   if (f && std::strcmp(f, "wide")) return false;
   if (!woq_wide_plan(a.M, a.N, a.K, a.G, p)) return false;
-  return a.x_dt == ZT_DT_BF16 && a.s_dt == ZT_DT_BF16 && !a.zp && a.ldx % 8 == 0 &&
-         aligned16(a.x) && aligned16(a.w) &&
+  // zero points: 8-bit, in whole dwords (N % 4 == 0 is in the plan)
+  if (a.zp && ((a.zp_dt != ZT_DT_S8 && a.zp_dt != ZT_DT_U8) ||
+               (reinterpret_cast<uintptr_t>(a.zp) & 3u)))
+    return false;
+  return a.x_dt == ZT_DT_BF16 && a.s_dt == ZT_DT_BF16 && a.ldx % 8 == 0 && aligned16(a.x) && aligned16(a.w) &&
          (a.M - 1) * a.ldx * 2 + a.K * 2 < (int64_t)kOobOffset &&
          a.N * (a.K / 2) < (int64_t)kOobOffset && a.G * a.N * 2 < (int64_t)kOobOffset;
 }
@@ -2893,24 +2984,71 @@ bool woq_try_stream(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   return try_launch_stream(a, s, shift, gmask, mode, err);
 }
 
+// The staged mode that takes a call's scales and zero points, or -1: bf16
+// scales in groups of 32 and up that are a power of two times 32 (or per
+// channel), no zero points or 8-bit ones, and the alignment of their DMA.
+// *shift: log2 of the blocks of 32 per group.
+static int group_mode(const WoqArgs &a, int *shift, int *gmask) {
+  const int64_t g32 = a.K / a.G / 32;
+  if (a.x_dt != ZT_DT_BF16 || a.s_dt != ZT_DT_BF16 || a.K % 128 || a.N % (a.zp ? 4 : 2) ||
+      (a.G > 1 && ((a.K / a.G) % 32 || (g32 & (g32 - 1)))) ||
+      (reinterpret_cast<uintptr_t>(a.scales) & 3u) || a.G * a.N * 2 >= (int64_t)kOobOffset)
+    return -1;
+  if (a.zp && ((a.zp_dt != ZT_DT_S8 && a.zp_dt != ZT_DT_U8) ||
+               (reinterpret_cast<uintptr_t>(a.zp) & 3u)))
+    return -1;
+  *gmask = a.G == 1 ? 0 : 0x7fffffff;
+  *shift = 0;
+  if (a.G > 1)
+    while (((int64_t)1 << *shift) < g32) ++*shift;
+  return a.zp ? kDecU4G : kDecS4G;
+}
+
+// Up to 64 rows with 8-bit zero points or in groups of 32 / 64 on the stream
+// kernel (false: not such a call, or no layout for it).  18944 x 3584 at M = 1 /
+// 8 / 16: with zero points 21.3 / 27.0 / 43.5 us in the general mode, 12.5 / 14.8 /
+// 20.3 here (signed 11.4 / 14.2 / 19.7); in groups of 64 26.9 / 27.3 / 27.9 on the
+// prefill kernel, 12.1 / 14.5 / 20.3 here.
+static bool group_stream(const WoqArgs &a, hipStream_t s, hipError_t *err, int *plan_p) {
+  int shift, gmask;
+  const int mode = group_mode(a, &shift, &gmask);
+  if (mode < 0 || a.M > 64 || a.ldx % 8 || !aligned16(a.x) || !aligned16(a.w) ||
+      a.N * (a.K / 2) >= (int64_t)kOobOffset)
+    return false;
+  if (mode == kDecS4G && (a.G == 1 || (a.K / a.G) % 128 == 0)) return false;  // the fast mode
+  return try_launch_stream(a, s, shift, gmask, mode, err, plan_p);
+}
+
+bool woq_try_group_stream(const WoqArgs &a, hipStream_t s, hipError_t *err) {
+  return group_stream(a, s, err, nullptr);
+}
+
+bool woq_group_stream_ok(const WoqArgs &a) {
+  hipError_t err = hipSuccess;
+  int p = 0;
+  return group_stream(a, nullptr, &err, &p);
+}
+
 // The merged gate_up launch of the stream kernel (fast mode, M <= 16, x
 // whole in LDS).  Returns false when the caller should take the two-step
 // path (the full linear into fp32, then launch_silu_mul_halves).
 bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   const int64_t I = a.N / 2, gs = a.K / a.G, cpg = gs / 128;
-  if (a.x_dt != ZT_DT_BF16 || a.s_dt != ZT_DT_BF16 || a.zp || a.M < 1 || a.M > 16 ||
-      a.N % 32 != 0 || a.K % 128 != 0 || (a.G != 1 && (gs % 128 || (cpg & (cpg - 1)))) ||
-      a.ldx % 8 != 0 || !aligned16(a.x) || !aligned16(a.w) ||
+  if (a.x_dt != ZT_DT_BF16 || a.s_dt != ZT_DT_BF16 || a.M < 1 || a.M > 16 || a.N % 32 != 0 ||
+      a.K % 128 != 0 || a.ldx % 8 != 0 || !aligned16(a.x) || !aligned16(a.w) ||
       a.N * (a.K / 2) >= (int64_t)kOobOffset || a.G * a.N * 2 >= (int64_t)kOobOffset)
     return false;
-  int shift = 0;
+  int shift = 0, gmask = a.G == 1 ? 0 : 0x7fffffff, mode = kDecFast;
   while (cpg > 1 && (1 << shift) < cpg) ++shift;
-  const int gmask = a.G == 1 ? 0 : 0x7fffffff;
-  if (!knob(kKnobWoqStream) && try_launch_lean(a, s, shift, gmask, kDecFast, (int)I, err))
+  if (a.zp || (a.G != 1 && (gs % 128 || (cpg & (cpg - 1))))) {
+    mode = group_mode(a, &shift, &gmask);
+    if (mode < 0) return false;
+  }
+  if (!knob(kKnobWoqStream) && try_launch_lean(a, s, shift, gmask, mode, (int)I, err))
     return true;
-  if (!knob(kKnobWoqStream) && try_launch_persist(a, s, shift, gmask, kDecFast, (int)I, err))
+  if (!knob(kKnobWoqStream) && try_launch_persist(a, s, shift, gmask, mode, (int)I, err))
     return true;
-  if (!knob(kKnobWoqStream) && try_launch_wave(a, s, shift, gmask, kDecFast, (int)I, err))
+  if (!knob(kKnobWoqStream) && try_launch_wave(a, s, shift, gmask, mode, (int)I, err))
     return true;
   const int C = (int)(a.K / 128), tiles = (int)(a.N / 16);
   const size_t x_bytes = (size_t)a.M * stream_x_pitch((int)a.K) * 2;
@@ -2928,7 +3066,7 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
     if (woq_wide_ok(a, &wp) && wp.splits == 1) return false;
   }
   const size_t lds = stream_scale_offset(stream_slab_bytes(8, tpw, 1), x_bytes) +
-                     stream_scale_bytes((int)a.G, tpw);
+                     stream_staged_bytes(mode, (int)a.G, tpw);
   if (lds > kStreamLdsMax) return false;
   const int need = (C + 7) / 8;
   int cpw = 0;
@@ -2940,16 +3078,21 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   if (knob(kKnobWoqDebug))
     std::fprintf(stderr, "[zt] woq gate_up stream M=%lld N=%lld K=%lld: CPW=%d TPW=%d\n",
                  (long long)a.M, (long long)a.N, (long long)a.K, cpw, tpw);
+#define ZT_GU_MODE(CPW_, TPW_, MODE_)                                                       \
+  woq_stream_kernel<8, CPW_, TPW_, MODE_, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask,  \
+                                                                        x_dma, (int)I)
 #define ZT_GU_CASE(CPW_, TPW_)                                                              \
   if (cpw == CPW_ && tpw == TPW_) {                                                        \
-    woq_stream_kernel<8, CPW_, TPW_, kDecFast, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask, \
-                                                                            x_dma, (int)I); \
+    if (mode == kDecFast) ZT_GU_MODE(CPW_, TPW_, kDecFast);                                \
+    else if (mode == kDecS4G) ZT_GU_MODE(CPW_, TPW_, kDecS4G);                             \
+    else ZT_GU_MODE(CPW_, TPW_, kDecU4G);                                                  \
     *err = hipGetLastError();                                                              \
     return true;                                                                           \
   }
   ZT_GU_CASE(4, 2) ZT_GU_CASE(8, 2) ZT_GU_CASE(14, 2) ZT_GU_CASE(16, 2)
   ZT_GU_CASE(2, 4) ZT_GU_CASE(4, 4) ZT_GU_CASE(8, 4)
 #undef ZT_GU_CASE
+#undef ZT_GU_MODE
   return false;
 }
 

@@ -75,12 +75,15 @@ size_t woq_gemm_workspace(int64_t M, int64_t N, int64_t K);
 // The weight-streaming decode kernel for up to 64 rows, when it applies
 // (returns false otherwise; *err holds the launch status when it does).
 bool woq_try_stream(const WoqArgs &a, hipStream_t s, hipError_t *err);
+// its form for 8-bit zero points and groups of 32 / 64
+bool woq_try_group_stream(const WoqArgs &a, hipStream_t s, hipError_t *err);
+bool woq_group_stream_ok(const WoqArgs &a);  // whether it would take the call
 // merged gate_up (weight rows [0, N/2) gate, [N/2, N) up): y = silu(gate) * up
 bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err);
 hipError_t launch_silu_mul_halves(const float *h, int64_t ld_h, int64_t M, int64_t I, void *y,
                                   int y_dt, int64_t ldy, hipStream_t s);
 // 17..64 rows: the wide weight-streaming kernel (bf16 x and scales, no
-// zero points), K split over `splits` workgroups per row block whose fp32
+// zero points or 8-bit ones), K split over `splits` workgroups per row block whose fp32
 // partials take woq_wide_workspace bytes of workspace.
 struct WidePlan {
   int mt;      // 32-token tiles (1 or 2)
