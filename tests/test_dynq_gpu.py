@@ -48,6 +48,19 @@ def test_quantize_bit_exact(M, K, x_dtype):
     assert torch.equal(qx.cpu(), qr)
 
 
+# rows of 2056 elements and more take 512 and 1024 threads at up to 256 rows
+# and 256 past them: the edges of each width, both sides of the row limit
+@pytest.mark.parametrize("K", [2048, 2056, 4096, 4104, 8192, 8200, 16392])
+@pytest.mark.parametrize("M", [1, 256, 257])
+@pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])
+def test_quantize_threads_per_row_bit_exact(M, K, x_dtype):
+    x = (torch.randn(M, K, generator=torch.Generator().manual_seed(M + K)) * 2).to(x_dtype)
+    qx, sx = C.dynamic_quantize(x.to(DEV))
+    qr, sr = O.dynamic_quantize(x)
+    assert torch.equal(sx.cpu(), sr)
+    assert torch.equal(qx.cpu(), qr)
+
+
 # quotients x / s that are exactly half-integers (ties, rounded to even) or
 # within an ulp of one: rows whose amax is 127 * 2^e make s = 2^e exact
 @pytest.mark.parametrize("x_dtype", [torch.bfloat16, torch.float32])

@@ -2215,10 +2215,13 @@ hipError_t launch_dyn_quantize(const void *x, int x_dt, int64_t M, int64_t K,
     return hipGetLastError();                                                              \
   }
     // Few rows: their workgroups do not fill the GPU, so a row's time is one
-    // thread's, and longer rows take more threads (8 x 14336: 5.8 us with 256)
-    const bool few = M <= 256 && per > 2;
+    // thread's, and rows past 2048 take more threads (8 x 14336: 5.8 us with
+    // 256; the 128 x 4096 linear call 20.2 us with 256, 19.8 with 512)
+    const bool few = M <= 256 && per > 1;
     if (x_dt == ZT_DT_BF16) {
-      if (few) { ZT_QV(Bf16x8, 1024, 1) ZT_QV(Bf16x8, 1024, 2) ZT_QV(Bf16x8, 1024, 4) }
+      if (few) {
+        ZT_QV(Bf16x8, 512, 1) ZT_QV(Bf16x8, 1024, 1) ZT_QV(Bf16x8, 1024, 2) ZT_QV(Bf16x8, 1024, 4)
+      }
       ZT_QV(Bf16x8, 256, 2) ZT_QV(Bf16x8, 256, 4) ZT_QV(Bf16x8, 256, 8) ZT_QV(Bf16x8, 256, 16)
     } else {
       if (few) { ZT_QV(F32x8, 1024, 1) ZT_QV(F32x8, 1024, 2) ZT_QV(F32x8, 1024, 4) }
