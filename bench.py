@@ -759,7 +759,7 @@ def secondary_rooflines(res):
                     "bound": "hbm", "achieved": round(d["GBps"], 2), "peak": HBM_PEAK_GBS,
                     "unit": "GB/s", "frac": round(d["frac_hbm"], 4),
                     "achieved_tops": round(d["TOPS"], 2), "frac_int8_peak": round(d["frac_int8_peak"], 4),
-                    "kernels": "dyn_quantize_bf16_kernel + s8_splitk_kernel",
+                    "kernels": "dyn_quantize_vec_kernel + s8_splitk_kernel",
                     "op_avg_us": round(d["s_per_call"] * 1e6, 3)})
     d = res.get("dyn_qlinear_asym_m128")
     if d:
@@ -785,7 +785,7 @@ def secondary_rooflines(res):
         out.append({"workload": "config 3 int8: dynamic qlinear over the Llama-3-8B layer, M=2048",
                     "bound": "mfma", "achieved": round(d["TOPS"], 2), "peak": INT8_PEAK_TOPS,
                     "unit": "TOP/s", "frac": round(d["frac_int8_peak"], 4),
-                    "kernels": "dyn_quantize_bf16_kernel + s8_gemm_ws_kernel",
+                    "kernels": "dyn_quantize_vec_kernel + s8_prefill_kernel / s8_gemm_ws_kernel",
                     "layer_avg_us": round(d["s_per_layer"] * 1e6, 3),
                     "weight_copies": d["weight_copies"]})
     d = res.get("prefill_int4_m2048")
@@ -793,7 +793,7 @@ def secondary_rooflines(res):
         out.append({"workload": "config 3 int4: WOQ linear over the Llama-3-8B layer, M=2048",
                     "bound": "mfma", "achieved": round(d["TFLOPS"], 2), "peak": BF16_PEAK_TFLOPS,
                     "unit": "TFLOP/s", "frac": round(d["frac_bf16_peak"], 4),
-                    "kernels": "woq_gemm_ws_kernel (qkv, o, down) + woq_gemm32_kernel (gate_up)",
+                    "kernels": "woq_prefill_kernel",
                     "layer_avg_us": round(d["s_per_layer"] * 1e6, 3),
                     "weight_copies": d["weight_copies"]})
     for d in res.get("decode_layer", []):

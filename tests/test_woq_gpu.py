@@ -218,9 +218,8 @@ def test_wide_kernel_strided_x():
     check_close(y, y_ref)
 
 
-# the 32x32 prefill kernel (bf16 scales, no zero points, N % 8 == 0):
-# 128 x 128 and 256 x 128 tiles, ragged M and N, group sizes 128 / 256 /
-# per-channel, more tiles than CUs
+# the default prefill kernels (bf16 scales, no zero points): ragged M and N,
+# group sizes 128 / 256 / per-channel, more tiles than CUs
 @pytest.mark.parametrize("M,K,N,G", [(300, 1024, 200, 8), (520, 512, 264, 2),
                                      (1100, 2048, 1032, 1), (2100, 768, 4104, 6)])
 def test_gemm32_kernel_vs_oracle(M, K, N, G):
@@ -600,12 +599,9 @@ def test_persist_kernel_gate_up_strided_x():
     assert torch.equal(y, y0)
 
 
-# every prefill GEMM variant by name (ZT_WOQ_GEMM): "1" the 32x32 kernel with
-# 128 x 128 tiles (256 x 128 is the default at this size), "w" / "v" its
-# load-wave form with 4 / 3 stages, "x" with 256 x 192 tiles (ragged in N
-# here), "d" the 16x16 DMA kernel, "2" its
-# 256 x 128 tiles, "o" the 16x16 kernel without DMA; ragged M and N, two
-# scale dtypes
+# every prefill GEMM variant by name (ZT_WOQ_GEMM): "w" / "v" / "x" the
+# load-wave kernel, "o" the synchronous kernel, any other the large-tile kernel
+# unsplit; ragged M and N, two scale dtypes
 @pytest.mark.parametrize("variant", ["1", "w", "v", "x", "d", "2", "o"])
 @pytest.mark.parametrize("M,K,N,G,s_dtype", [(300, 1024, 264, 8, torch.bfloat16),
                                              (520, 2048, 520, 16, torch.bfloat16),
@@ -619,9 +615,8 @@ def test_prefill_gemm_variants(variant, M, K, N, G, s_dtype):
     check_close(y, y_ref)
 
 
-# post-ops in the prefill variants' epilogues: the 32x32 kernel ("1"), its
-# load-wave form with 256 x 128 and 256 x 192 tiles ("w", "x") and the
-# 16x16 DMA kernel ("2"), with bias, elementwise and binary post-ops
+# post-ops in the prefill variants' epilogues (the large-tile and the load-wave
+# kernel), with bias, elementwise and binary post-ops
 @pytest.mark.parametrize("variant", ["1", "w", "x", "2"])
 @pytest.mark.parametrize("post,nbuf", [(("gelu_erf",), 0), (("mul", "add"), 2),
                                        (("silu", "mul"), 1)])
@@ -637,8 +632,7 @@ def test_prefill_variants_post_ops(variant, post, nbuf):
     check_close(y, y_ref)
 
 
-# the default prefill dispatch at one round of 256 x 128 tiles (128 tiles
-# here) takes the load-wave kernel
+# the default prefill dispatch at half a round of 256 x 128 tiles
 def test_prefill_one_round_default_kernel():
     M, K, N, G = 2048, 256, 2048, 2
     x, q, wp, s, z, b = make_case(M, K, N, G, seed=11, bias=True)
@@ -648,8 +642,7 @@ def test_prefill_one_round_default_kernel():
     check_close(y, y_ref)
 
 
-# 256 x 192 tiles by default where they make one round and 256 x 128 do not:
-# 9 x 24 = 216 tiles of 256 x 192 against 9 x 36 = 324 of 256 x 128 (ragged M)
+# ragged M over more than one round of 256 x 128 tiles (9 x 36 = 324)
 def test_prefill_one_round_192_default_kernel():
     M, K, N, G = 2100, 256, 4608, 2
     x, q, wp, s, z, b = make_case(M, K, N, G, seed=12, bias=True)

@@ -35,9 +35,9 @@
 //    and 64.
 //  * woq_gemm_ws_kernel  one nearly full round of 256 x 128 tiles at up to
 //    512 rows (signed int4, bf16 scales): loads in waves of their own, three
-//    stages.  woq_gemm32_kernel / woq_gemm_dma_kernel / woq_gemm_kernel: the
-//    kernels before woq_prefill_kernel, selectable, and for what its 32-bit
-//    offsets and group sizes exclude.
+//    stages.
+//  * woq_gemm_kernel  synchronous tiles for what the 32-bit offsets, x types,
+//    alignment and group sizes of woq_prefill_kernel exclude.
 //  * woq_generic_kernel  what none of the above takes (K not a multiple of
 //    64, odd group sizes): one wave per output element.
 //
@@ -685,31 +685,7 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
   }
 }
 
-// ----------------------------------------------------- prefill GEMM (DMA)
-// BM x BN output tile, 4 waves (2 x 2) of (BM/2) x (BN/2), K in steps of
-// 128.  Per step the buffer unit moves straight into LDS:
-//  * the x slab [BM, 128] bf16: 256-byte rows whose sixteen 16-byte chunks
-//    are XOR-swizzled (chunk c of row r at position c ^ (r & 15)), so the 16
-//    rows of a fragment read hit every bank once;
-//  * the raw int4 slab [BN, 128] (64-byte rows of packed words).
-// A lane's B operand for a step is one 16-byte read (the 32 elements
-// [32g, 32g+32) of its row, g = lane / 16), dequantised in registers right
-// before its MFMAs -- exactly bf16_rne of the reference's fp32 dequantised
-// weight -- and its A operand for sub-step i is the 16 bytes of x at element
-// 32g + 8i, the same element order.  Two LDS stages; the step's reads are
-// issued before the next step's loads, the MFMAs after, one barrier a step.
-// The fp32 tile is staged in LDS for the epilogue (bias, post-ops, 8-byte
-// bf16 stores).
-constexpr int kXRow = 256;   // bytes of x per row per step
-constexpr int kWRow = 64;    // bytes of int4 per weight row per step
-
-template <int BM, int BN>
-constexpr size_t woq_dma_lds() {
-  const size_t stages = 2 * ((size_t)BM * kXRow + (size_t)BN * kWRow);
-  const size_t tile = (size_t)BM * (BN + 4) * 4;
-  return stages > tile ? stages : tile;
-}
-
+// ------------------------------------------- prefill GEMM, load waves
 // Epilogue of ROWS x BN fp32 outputs staged in LDS (row pitch BN + 4) for
 // rows m0.. and columns n0..: bias, post-ops, then rows of four columns per
 // thread (8-byte bf16 stores where the row allows), NT threads.
@@ -746,168 +722,18 @@ __device__ __forceinline__ void woq_tile_epilogue(const WoqArgs &a, const float 
   }
 }
 
-template <int BM, int BN, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1)))
-void woq_gemm_dma_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int cpg_shift,
-                         int gmask) {
-  constexpr int WTM = BM / 32, WTN = BN / 32;
-  constexpr int STAGE = BM * kXRow + BN * kWRow;
-  constexpr int XI = BM * kXRow / 1024;  // 1 KB loads per stage: x
-  constexpr int WI = BN * kWRow / 1024;  //                        weights
-  static_assert((XI + WI) % 4 == 0, "loads must split over 4 waves");
-  constexpr int LPW = (XI + WI) / 4;
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wv >> 1, wn = wv & 1;
-  const int lr = lane & 15, lg = lane >> 4;
-
-  const int t = xcd_contiguous_tile(blockIdx.x, tiles_m * tiles_n);
-  const int per_group = group_m * tiles_n;
-  const int g = t / per_group, tg = t - g * per_group;
-  const int gm = min(group_m, tiles_m - g * group_m);
-  const int tm = g * group_m + tg % gm, tn = tg / gm;
-  const int M = (int)a.M, N = (int)a.N, K = (int)a.K;
-  const int KW = K / 8;
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int zmode = zp_mode_of(a.zp, a.zp_dt);
-  const int s_bytes = MODE == kDecGenF32 ? 4 : 2;
-
-  const auto x_rs = make_rsrc(a.x, (uint32_t)((int64_t)M * a.ldx * 2));
-  const auto w_rs = make_rsrc(a.w, (uint32_t)((int64_t)N * KW * 4));
-  const auto s_rs = make_rsrc(a.scales, (uint32_t)(a.G * N * s_bytes));
-
-  // This wave's LPW 1 KB loads per stage: x loads cover 4 rows (16 lanes x
-  // 16 B each, chunk positions XOR-swizzled by row), weight loads 16 rows
-  // (4 lanes x 16 B each).
-  const int ldx2 = (int)a.ldx * 2;
-  auto dma = [&](int step) {
-    unsigned char *stage = smem + (step & 1) * STAGE;
-#pragma unroll
-    for (int q = 0; q < LPW; ++q) {
-      const int li = wv * LPW + q;
-      if (li < XI) {
-        const int row = li * 4 + (lane >> 4);
-        const int chunk = (lane & 15) ^ (row & 15);
-        const uint32_t off = m0 + row < M ? (uint32_t)((m0 + row) * ldx2 + step * kXRow + chunk * 16)
-                                          : kOobOffset;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rs, (lds_ptr_t)(stage + li * 1024), 16, off, 0, 0, 0);
-      } else {
-        const int wi = li - XI;
-        const int row = wi * 16 + (lane >> 2);
-        const uint32_t off = n0 + row < N ? (uint32_t)((n0 + row) * KW * 4 + step * kWRow + (lane & 3) * 16)
-                                          : kOobOffset;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rs, (lds_ptr_t)(stage + BM * kXRow + wi * 1024), 16,
-                                                 off, 0, 0, 0);
-      }
-    }
-  };
-
-  // this lane's weight rows (clamped: rows past N are computed, never stored)
-  uint32_t srow[WTN];
-#pragma unroll
-  for (int j = 0; j < WTN; ++j) srow[j] = (uint32_t)min(n0 + wn * (BN / 2) + j * 16 + lr, N - 1);
-
-  f32x4_t acc[WTM][WTN];
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) acc[i][j] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-  const int nk = K / 128;
-  dma(0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  for (int ks = 0; ks < nk; ++ks) {
-    const unsigned char *stage = smem + (ks & 1) * STAGE;
-    // scales (and zero points) of this step, one per weight row
-    uint32_t sraw[WTN];
-    float zr[WTN];
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) {
-      const uint32_t sidx = (uint32_t)((ks >> cpg_shift) & gmask) * (uint32_t)N + srow[j];
-      sraw[j] = MODE == kDecGenF32 ? __builtin_amdgcn_raw_buffer_load_b32(s_rs, sidx * 4u, 0, 0)
-                                   : __builtin_amdgcn_raw_buffer_load_b16(s_rs, sidx * 2u, 0, 0);
-      zr[j] = (MODE != kDecFast && zmode) ? load_elem(a.zp, a.zp_dt, sidx) : 0.f;
-    }
-    // raw weight words: row (wn*BN/2 + j*16 + lr), 16 bytes at 16*lg
-    u32x4_t wraw[WTN];
-#pragma unroll
-    for (int j = 0; j < WTN; ++j)
-      wraw[j] = *reinterpret_cast<const u32x4_t *>(
-          stage + BM * kXRow + (wn * (BN / 2) + j * 16 + lr) * kWRow + 16 * lg);
-    // x fragments of all four sub-steps: row (wm*BM/2 + i*16 + lr), logical
-    // chunk 4*lg + sub (element 32*lg + 8*sub), swizzled by the row
-    u32x4_t xf[4][WTM];
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub)
-#pragma unroll
-      for (int i = 0; i < WTM; ++i) {
-        const int row = wm * (BM / 2) + i * 16 + lr;
-        xf[sub][i] = *reinterpret_cast<const u32x4_t *>(
-            stage + row * kXRow + (((4 * lg + sub) ^ (row & 15)) * 16));
-      }
-    if (ks + 1 < nk) dma(ks + 1);
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub) {
-      bf16x8_t B[WTN];
-#pragma unroll
-      for (int j = 0; j < WTN; ++j) {
-        const float sc = MODE == kDecGenF32 ? __uint_as_float(sraw[j]) : __uint_as_float(sraw[j] << 16);
-        B[j] = dq_word<MODE>(wraw[j][sub], sc, zr[j], zmode);
-      }
-#pragma unroll
-      for (int i = 0; i < WTM; ++i)
-#pragma unroll
-        for (int j = 0; j < WTN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
-              __builtin_bit_cast(bf16x8_t, xf[sub][i]), B[j], acc[i][j], 0, 0, 0);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-
-  // D[m = 4g + r][n = lane % 16] -> fp32 tile in LDS -> rows of 4 columns
-  constexpr int TP = BN + 4;
-  float *tile = reinterpret_cast<float *>(smem);
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r)
-        tile[(wm * (BM / 2) + i * 16 + 4 * lg + r) * TP + wn * (BN / 2) + j * 16 + lr] = acc[i][j][r];
-  __syncthreads();
-  woq_tile_epilogue<BM, BN>(a, tile, m0, n0, tid);
-}
-
-// ROWS x BN fp32 tile staged in LDS (row pitch BN + 4) -> rows m0.. and
-// columns n0.. of a K split's fp32 partial [M][N] (N % 4 == 0: a column
-// quad lies wholly inside or past N), NT threads.
-template <int ROWS, int BN, int NT = 256>
-__device__ __forceinline__ void woq_tile_store_partial(const float *tile, float *pp, int m0,
-                                                       int n0, int M, int N, int tid) {
-  constexpr int TP = BN + 4, Q = BN / 4;
-  for (int idx = tid; idx < ROWS * Q; idx += NT) {
-    const int r = idx / Q, c = (idx - r * Q) * 4;
-    const int m = m0 + r, n = n0 + c;
-    if (m < M && n < N)
-      *reinterpret_cast<f32x4_t *>(pp + (size_t)m * N + n) =
-          *reinterpret_cast<const f32x4_t *>(tile + r * TP + c);
-  }
-}
-
-// Prefill int4 GEMM on v_mfma_f32_32x32x16_bf16 (signed int4, bf16 scales):
-// BM x BN tiles, 4 waves of (BM/2) x (BN/2), K in steps of 64, two stages
-// moved straight into LDS by the buffer unit: the x slab [BM][64] bf16 (128 B
-// rows, 16-byte chunk c of row r at position c ^ ((r ^ (r >> 3)) & 7)), the
-// int4 slab [BN][64] (32 B rows, 16-byte half h of row r at h ^ ((r >> 3) &
-// 1)) and the step's scale row [BN] bf16.  Both swizzles give the 16 rows one
-// fragment read touches 16 distinct 16-byte bank groups.  Two workgroups per
-// CU (at most 256 registers and 80 KB of LDS each) overlap one another's
-// barriers and epilogues.
+// Prefill int4 GEMM on v_mfma_f32_32x32x16_bf16 (signed int4, bf16 scales)
+// with the loads in waves of their own: BM x BN tiles, K in steps of 64.  Four
+// compute waves of (BM/2) x (BN/2) only read LDS, dequantise and issue MFMAs;
+// four load waves move the S-stage slabs by DMA, S - 1 steps ahead, one
+// workgroup per CU: the x slab [BM][64] bf16 (128 B rows, 16-byte chunk c of
+// row r at position c ^ ((r ^ (r >> 3)) & 7)), the int4 slab [BN][64] (32 B
+// rows, 16-byte half h of row r at h ^ ((r >> 3) & 1)) and the step's scale
+// row [BN] bf16.  Both swizzles give the 16 rows one fragment read touches 16
+// distinct 16-byte bank groups.  A load wave waits only for its own loads
+// (in-order vmcnt); one s_barrier per step.  Every load wave issues the same
+// number of loads per step (the last ones out of range into a spare 1 KB of
+// LDS), so the wait count is one immediate.
 //
 // k order: the MFMA pairs A and B by k position, so any permutation shared
 // by both operands leaves the sums unchanged (bit for bit: each MFMA adds
@@ -920,10 +746,6 @@ __device__ __forceinline__ void woq_tile_store_partial(const float *tile, float 
 // weight), B = x, so D is [n][m]: register r of lane l holds
 // n = 8*(r/4) + 4*(l/32) + r%4 and m = l%32.  The epilogue stages one half of
 // the tile (the rows of the waves with wm == h) as fp32 [m][n] at a time.
-// With a K split (partial set, grid.y splits of sps steps) a workgroup walks
-// its split's steps only and writes its fp32 tile to partial[split][M][N];
-// woq_splitk_reduce_kernel then adds the splits in order and applies the
-// epilogue.
 constexpr int kW32BK = 64;
 
 // s_waitcnt immediate that waits for at most n outstanding vector-memory
@@ -933,169 +755,12 @@ __host__ __device__ constexpr int vmcnt_imm_woq(int n) {
 }
 
 template <int BM, int BN>
-constexpr size_t woq_gemm32_stage() {
+constexpr size_t woq_gemm_ws_stage() {
   return (size_t)BM * 128 + (size_t)BN * 32 + 1024;
 }
-template <int BM, int BN>
-constexpr size_t woq_gemm32_lds() {
-  const size_t stages = 2 * woq_gemm32_stage<BM, BN>();
-  const size_t half = (size_t)(BM / 2) * (BN + 4) * 4;
-  return stages > half ? stages : half;
-}
-
-template <int BM, int BN>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
-void woq_gemm32_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int cpg_shift,
-                       int gmask, float *partial, int sps) {
-  constexpr int WTM = BM / 64, WTN = BN / 64;  // 32 x 32 tiles per wave
-  constexpr int STAGE = (int)woq_gemm32_stage<BM, BN>();
-  constexpr int XI = BM / 8;                    // 1 KB x loads (8 rows) per stage
-  constexpr int WI = BN / 32;                   // 1 KB weight loads (32 rows)
-  constexpr int LOADS = XI + WI + 1;            // + the scale row
-  constexpr int LPW = (LOADS + 3) / 4;
-  static_assert(BN <= 512 && BN % 64 == 0 && BM % 64 == 0, "tile shape");
-  extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wv >> 1, wn = wv & 1;
-  const int hl = lane >> 5, l32 = lane & 31;
-
-  const int t = xcd_contiguous_tile(blockIdx.x, tiles_m * tiles_n);
-  const int per_group = group_m * tiles_n;
-  const int g = t / per_group, tg = t - g * per_group;
-  const int gm = min(group_m, tiles_m - g * group_m);
-  const int tm = g * group_m + tg % gm, tn = tg / gm;
-  const int M = (int)a.M, N = (int)a.N, K = (int)a.K;
-  const int m0 = tm * BM, n0 = tn * BN;
-  const int ldx2 = (int)a.ldx * 2, KB = K / 2;
-
-  const auto x_rs = make_rsrc(a.x, (uint32_t)((int64_t)M * ldx2));
-  const auto w_rs = make_rsrc(a.w, (uint32_t)((int64_t)N * KB));
-  const auto s_rs = make_rsrc(a.scales, (uint32_t)(a.G * N * 2));
-
-  // the wave's loads: index li = wv * LPW + q; x loads first, then the
-  // weight loads, then the scale row (lanes 0..BN/8-1, 16 bytes each)
-  const int nk = K / kW32BK;
-  const int kb = partial ? (int)blockIdx.y * sps : 0;   // this workgroup's steps [kb, ke)
-  const int ke = partial ? min(kb + sps, nk) : nk;
-  auto dma = [&](int step) {
-    const int k0 = step * kW32BK;
-    const bool in = step < ke;
-    unsigned char *stage = smem + (step & 1) * STAGE;
-#pragma unroll
-    for (int q = 0; q < LPW; ++q) {
-      const int li = wv * LPW + q;
-      if (li >= LOADS) break;
-      uint32_t off;
-      if (li < XI) {
-        const int row = li * 8 + (lane >> 3);
-        const int chunk = (lane & 7) ^ ((row ^ (row >> 3)) & 7);
-        off = in && m0 + row < M ? (uint32_t)((m0 + row) * ldx2 + k0 * 2 + chunk * 16) : kOobOffset;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(x_rs, (lds_ptr_t)(stage + li * 1024), 16, off, 0, 0, 0);
-      } else if (li < XI + WI) {
-        const int wi = li - XI;
-        const int row = wi * 32 + (lane >> 1);
-        const int half = (lane & 1) ^ ((row >> 3) & 1);
-        off = in && n0 + row < N ? (uint32_t)((n0 + row) * KB + k0 / 2 + half * 16) : kOobOffset;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(w_rs, (lds_ptr_t)(stage + BM * 128 + wi * 1024), 16,
-                                                 off, 0, 0, 0);
-      } else {
-        // N % 8 == 0 (host-checked): a lane's 8 scales lie wholly inside or past N
-        const uint32_t grp = (uint32_t)(((k0 >> 7) >> cpg_shift) & gmask);
-        off = in && lane < BN / 8 && n0 + 8 * lane < N
-                  ? (grp * (uint32_t)N + (uint32_t)(n0 + 8 * lane)) * 2u
-                  : kOobOffset;
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(s_rs, (lds_ptr_t)(stage + BM * 128 + BN * 32), 16,
-                                                 off, 0, 0, 0);
-      }
-    }
-  };
-
-  f32x16_t acc[WTM][WTN];
-#pragma unroll
-  for (int i = 0; i < WTM; ++i)
-#pragma unroll
-    for (int j = 0; j < WTN; ++j)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-  dma(kb);
-  for (int ks = kb; ks < ke; ++ks) {
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): this wave's loads of step ks
-    asm volatile("s_barrier" ::: "memory");
-    dma(ks + 1);  // past the last step: zeros into the buffer step ks - 1 used
-    const unsigned char *stage = smem + (ks & 1) * STAGE;
-    // weight words 4h..4h+3 of rows wn*BN/2 + 32j + l32, and their scales
-    u32x4_t wq[WTN];
-    float sc[WTN];
-#pragma unroll
-    for (int j = 0; j < WTN; ++j) {
-      const int row = wn * (BN / 2) + j * 32 + l32;
-      wq[j] = *reinterpret_cast<const u32x4_t *>(stage + BM * 128 + row * 32 +
-                                                 ((hl ^ ((row >> 3) & 1)) * 16));
-      sc[j] = bf16_bits_to_f32(
-          *reinterpret_cast<const uint16_t *>(stage + BM * 128 + BN * 32 + row * 2));
-    }
-#pragma unroll
-    for (int sub = 0; sub < 4; ++sub) {
-      const int chunk = 4 * hl + sub;
-      bf16x8_t xb[WTM];
-#pragma unroll
-      for (int i = 0; i < WTM; ++i) {
-        const int row = wm * (BM / 2) + i * 32 + l32;
-        xb[i] = *reinterpret_cast<const bf16x8_t *>(stage + row * 128 +
-                                                    ((chunk ^ ((row ^ (row >> 3)) & 7)) * 16));
-      }
-#pragma unroll
-      for (int j = 0; j < WTN; ++j) {
-        const bf16x8_t wb = dq_word<kDecFast>(wq[j][sub], sc[j], 0.f, 0);
-#pragma unroll
-        for (int i = 0; i < WTM; ++i)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wb, xb[i], acc[i][j], 0, 0, 0);
-      }
-    }
-  }
-
-  // epilogue in two halves of BM/2 rows
-  __builtin_amdgcn_s_waitcnt(0);
-  asm volatile("s_barrier" ::: "memory");
-  constexpr int TP = BN + 4;
-  float *tile = reinterpret_cast<float *>(smem);
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    if (wm == h) {
-#pragma unroll
-      for (int i = 0; i < WTM; ++i)
-#pragma unroll
-        for (int j = 0; j < WTN; ++j)
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            *reinterpret_cast<f32x4_t *>(tile + (i * 32 + l32) * TP + wn * (BN / 2) + j * 32 + 8 * q +
-                                         4 * hl) =
-                f32x4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2],
-                        acc[i][j][4 * q + 3]};
-    }
-    __syncthreads();
-    if (partial)
-      woq_tile_store_partial<BM / 2, BN>(tile, partial + (size_t)blockIdx.y * M * N,
-                                         m0 + h * (BM / 2), n0, M, N, tid);
-    else
-      woq_tile_epilogue<BM / 2, BN>(a, tile, m0 + h * (BM / 2), n0, tid);
-    __syncthreads();
-  }
-}
-
-// The same tile with the loads in waves of their own (as s8_gemm_ws_kernel
-// does for int8): four compute waves (128 x 64 each) only read LDS, dequantise
-// and issue MFMAs; four load waves move the S-stage [x | W | scales] slabs
-// by DMA, S - 1 steps ahead, one workgroup per CU.  A load wave waits only
-// for its own loads (in-order vmcnt); one s_barrier per step.  Every load
-// wave issues the same number of loads per step (the last ones out of range
-// into a spare 1 KB of LDS), so the wait count is one immediate.
 template <int BM, int BN, int S>
 constexpr size_t woq_gemm_ws_lds() {
-  const size_t stages = (size_t)S * woq_gemm32_stage<BM, BN>() + 1024;
+  const size_t stages = (size_t)S * woq_gemm_ws_stage<BM, BN>() + 1024;
   const size_t half = (size_t)(BM / 2) * (BN + 4) * 4;
   return stages > half ? stages : half;
 }
@@ -1105,7 +770,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void woq_gemm_ws_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int cpg_shift,
                         int gmask) {
   constexpr int WTM = BM / 64, WTN = BN / 64;  // 32 x 32 tiles per compute wave
-  constexpr int STAGE = (int)woq_gemm32_stage<BM, BN>();
+  constexpr int STAGE = (int)woq_gemm_ws_stage<BM, BN>();
   constexpr int XI = BM / 8;          // 1 KB x loads (8 rows) per stage
   constexpr int WI = BN / 32;         // 1 KB weight loads (32 rows)
   constexpr int LOADS = XI + WI + 1;  // + the scale row
@@ -1252,36 +917,6 @@ static hipError_t launch_woq_gemm_ws_t(const WoqArgs &a, hipStream_t s, int shif
   woq_gemm_ws_kernel<BM, BN, S><<<dim3((unsigned)(tiles_m * tiles_n)), dim3(512),
                                   woq_gemm_ws_lds<BM, BN, S>(), s>>>(a, tiles_m, tiles_n, group_m,
                                                                      shift, gmask);
-  return hipGetLastError();
-}
-
-// splits > 1: K split into splits ranges of whole steps, fp32 partials to
-// `partial` ([splits][M][N]); the caller adds them
-template <int BM, int BN>
-static hipError_t launch_woq_gemm32_t(const WoqArgs &a, hipStream_t s, int shift, int gmask,
-                                      float *partial = nullptr, int splits = 1) {
-  const int tiles_m = (int)((a.M + BM - 1) / BM), tiles_n = (int)((a.N + BN - 1) / BN);
-  const int group_m = tiles_m < 4 ? tiles_m : 4;
-  const int nk = (int)(a.K / kW32BK);
-  const int sps = splits > 1 ? (nk + splits - 1) / splits : nk;
-  woq_gemm32_kernel<BM, BN><<<dim3((unsigned)(tiles_m * tiles_n), (unsigned)(splits > 1 ? splits : 1)),
-                              dim3(256), woq_gemm32_lds<BM, BN>(), s>>>(
-      a, tiles_m, tiles_n, group_m, shift, gmask, splits > 1 ? partial : nullptr, sps);
-  return hipGetLastError();
-}
-
-template <int BM, int BN>
-static hipError_t launch_woq_dma_t(const WoqArgs &a, hipStream_t s, int shift, int gmask, int mode) {
-  const int tiles_m = (int)((a.M + BM - 1) / BM), tiles_n = (int)((a.N + BN - 1) / BN);
-  const int group_m = tiles_m < 4 ? tiles_m : 4;
-  dim3 grid((unsigned)(tiles_m * tiles_n)), block(256);
-  const size_t lds = woq_dma_lds<BM, BN>();
-  if (mode == kDecFast)
-    woq_gemm_dma_kernel<BM, BN, kDecFast><<<grid, block, lds, s>>>(a, tiles_m, tiles_n, group_m, shift, gmask);
-  else if (mode == kDecGenBf16)
-    woq_gemm_dma_kernel<BM, BN, kDecGenBf16><<<grid, block, lds, s>>>(a, tiles_m, tiles_n, group_m, shift, gmask);
-  else
-    woq_gemm_dma_kernel<BM, BN, kDecGenF32><<<grid, block, lds, s>>>(a, tiles_m, tiles_n, group_m, shift, gmask);
   return hipGetLastError();
 }
 
@@ -3178,81 +2813,26 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {
 }
 
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace, size_t workspace_bytes) {
-  const char *forced = knob(kKnobWoqGemm);
-  // The large-tile kernel, except where the load-wave kernel below is still
-  // ahead: one round of its 256 x 128 tiles at least three quarters full over
-  // at most two row tiles, where the weights come from HBM and its third
-  // stage hides more of that (signed int4 with bf16 scales; 28672 x 4096 at
-  // M = 256 70.4 against 73-77 us, 16384 x 3072 at M = 512 57 against 60).
-  const int64_t lw_tiles = ((a.M + 255) / 256) * ((a.N + 127) / 128);
-  const bool load_wave = a.M <= 512 && lw_tiles > 192 && lw_tiles <= 256 && !a.zp &&
-                         a.s_dt == ZT_DT_BF16 && a.N % 8 == 0 && a.K % 128 == 0 &&
-                         (a.G == 1 || (a.K / a.G) % 128 == 0);
-  if (a.M > 0 && a.N > 0 && (forced ? forced[0] == 'p' : !load_wave) && woq_prefill_ok(a))
-    return launch_woq_prefill(a, false, workspace, workspace_bytes, s);
-  {
-    // the DMA kernel: bf16 x, K % 128 == 0, one scale per 128-chunk, 32-bit
-    // byte offsets for x and the weights
-    const int64_t gs = a.K / a.G, cpg = gs / 128;
-    const bool ok = a.x_dt == ZT_DT_BF16 && a.K % 128 == 0 && a.ldx % 8 == 0 &&
-                    aligned16(a.x) && aligned16(a.w) &&
-                    (a.G == 1 || (gs % 128 == 0 && (cpg & (cpg - 1)) == 0)) &&
-                    a.M * a.ldx * 2 < (int64_t)kOobOffset &&
-                    a.N * (a.K / 2) < (int64_t)kOobOffset;
-    const char *e = knob(kKnobWoqGemm);  // o: 16x16, d: 16x16 DMA, 1: 128x128, 2, w / v / x: load waves
-    if (ok && !(e && e[0] == 'o')) {
-      int shift = 0;
-      while (cpg > 1 && (1 << shift) < cpg) ++shift;
-      const int gmask = a.G == 1 ? 0 : 0x7fffffff;
-      const int mode = a.s_dt == ZT_DT_F32 ? kDecGenF32 : (a.zp ? kDecGenBf16 : kDecFast);
-      const int64_t t256 = ((a.M + 255) / 256) * ((a.N + 127) / 128);
-      // the 32x32 kernel: fast mode, K in 64-steps, scale rows of whole
-      // 16-byte pieces
-      if (mode == kDecFast && a.N % 8 == 0 && !(e && e[0] == 'd') &&
-          (int64_t)a.G * a.N * 2 < (int64_t)kOobOffset) {
-        // one round of 256 x 128 tiles (at most one per CU, more than half
-        // of them): the load-wave kernel, whose deeper prefetch is then not
-        // paid for by an epilogue that a second workgroup per CU would hide
-        // (O and down at M = 2048: 104 -> 81 and 327 -> 255 us); when 256 x
-        // 192 tiles make one round where 256 x 128 do not, those (QKV: 152 ->
-        // 112 us); more rounds: two workgroups per CU (gate_up 508 against 549
-        // us with 256 x 128).  At half a round or less the split path below
-        // (8192 x 8192 / 8192 x 28672 at M = 384: 106.8 / 338 us on 128
-        // load-wave tiles, 87.0 / 265 split in two)
-        const bool big32 = e ? e[0] != '1' : t256 > 128;
-        const bool ws = e ? e[0] == 'w' || e[0] == 'v' : t256 > 128 && t256 <= 256;
-        const int64_t t192 = ((a.M + 255) / 256) * ((a.N + 191) / 192);
-        const bool ws192 = e ? e[0] == 'x' : t256 > 256 && t192 <= 256;
-        if (ws192) return launch_woq_gemm_ws_t<256, 192, 3>(a, s, shift, gmask);
-        if (ws)
-          return e && e[0] == 'w' ? launch_woq_gemm_ws_t<256, 128, 4>(a, s, shift, gmask)
-                                  : launch_woq_gemm_ws_t<256, 128, 3>(a, s, shift, gmask);
-        if (big32) return launch_woq_gemm32_t<256, 128>(a, s, shift, gmask);
-        // few tiles: K split over fp32 partials in the workspace when it has
-        // room (graph replays over rotating weights, one box, M = 512:
-        // 4096 x 11008 148.5 us and 3072 x 8192 113.9 us unsplit, as long as
-        // at M = 2048 on twice the tile area)
-        const int sp = woq_gemm_splits(a.M, a.N, a.K);
-        const size_t need = woq_gemm_workspace(a.M, a.N, a.K);
-        if (sp > 1 && workspace && workspace_bytes >= need &&
-            (reinterpret_cast<uintptr_t>(workspace) & 15u) == 0) {
-          if (knob(kKnobWoqDebug))
-            std::fprintf(stderr, "[zt] woq gemm32 M=%lld N=%lld K=%lld: 128x128 tiles, %d K splits\n",
-                         (long long)a.M, (long long)a.N, (long long)a.K, sp);
-          float *partial = static_cast<float *>(workspace);
-          hipError_t err = launch_woq_gemm32_t<128, 128>(a, s, shift, gmask, partial, sp);
-          if (err != hipSuccess) return err;
-          return launch_splitk_reduce(a, partial, sp, s);
-        }
-        return launch_woq_gemm32_t<128, 128>(a, s, shift, gmask);
-      }
-      // 256 x 128 only for the fast mode: the general dequant spills there
-      const bool big = mode == kDecFast && (e ? e[0] == '2' : t256 >= 128);
-      return big ? launch_woq_dma_t<256, 128>(a, s, shift, gmask, mode)
-                 : launch_woq_dma_t<128, 128>(a, s, shift, gmask, mode);
-    }
-  }
   if (a.M == 0 || a.N == 0) return hipSuccess;
+  // o: the synchronous kernel, v / w / x: load waves, else the large tiles
+  const char *e = knob(kKnobWoqGemm);
+  if (woq_prefill_ok(a) && !(e && e[0] == 'o')) {
+    // The load-wave kernel where it is ahead of the large-tile kernel: one
+    // round of its 256 x 128 tiles at least three quarters full over at most
+    // two row tiles, where the weights come from HBM and its third stage hides
+    // more of that (signed int4 with bf16 scales; 28672 x 4096 at M = 256 70.4
+    // against 73-77 us, 16384 x 3072 at M = 512 57 against 60).  It needs one
+    // scale per 128-chunk and scale rows of whole 16-byte pieces.
+    const int64_t cpg = a.K / a.G / 128, tiles = ((a.M + 255) / 256) * ((a.N + 127) / 128);
+    const bool ok = !a.zp && a.s_dt == ZT_DT_BF16 && a.N % 8 == 0 && a.K % 128 == 0 &&
+                    (a.G == 1 || (a.K / a.G) % 128 == 0);
+    const bool load_wave = e ? e[0] == 'v' || e[0] == 'w' || e[0] == 'x'
+                             : a.M <= 512 && tiles > 192 && tiles <= 256;
+    if (!ok || !load_wave) return launch_woq_prefill(a, false, workspace, workspace_bytes, s);
+    int shift = 0;
+    while (cpg > 1 && (1 << shift) < cpg) ++shift;
+    return launch_woq_gemm_ws_t<256, 128, 3>(a, s, shift, a.G == 1 ? 0 : 0x7fffffff);
+  }
   if (a.M <= 64) {
     dim3 grid((unsigned)((a.N + 31) / 32), (unsigned)((a.M + 63) / 64));
     hipLaunchKernelGGL((woq_gemm_kernel<64, 32>), grid, dim3(256), 0, s, a);
