@@ -427,6 +427,13 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   hipError_t err = hipSuccess;
   if (zt::woq_try_stream_gate_up(a, s, &err)) return hip_status(err, op);
   if (zt::woq_try_wide_gate_up(a, s, &err)) return hip_status(err, op);
+  // the full [M, N] in fp32, asked of every call past the decode kernels:
+  // whether a shape needs it is not the caller's to know
+  const size_t h = ((size_t)M * (size_t)N * sizeof(float) + 255) / 256 * 256;
+  if (!workspace || workspace_bytes < h)
+    return fail(ZT_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op,
+                zt_woq_linear_gate_up_workspace_size(M, K, N, G),
+                workspace ? workspace_bytes : (size_t)0);
   // the prefill kernel's merged form past 64 rows, and where the plain linear
   // would take that kernel too; the decode kernels keep the two steps
   const char *forced = zt::knob(zt::kKnobWoqGemm);
@@ -439,11 +446,6 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
     return hip_status(zt::launch_woq_prefill(a, true, nullptr, 0, s), op);
   // two steps: the full [M, N] linear in fp32 into the workspace, then
   // silu(gate) * up over its halves
-  const size_t h = ((size_t)M * (size_t)N * sizeof(float) + 255) / 256 * 256;
-  if (!workspace || workspace_bytes < h)
-    return fail(ZT_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op,
-                zt_woq_linear_gate_up_workspace_size(M, K, N, G),
-                workspace ? workspace_bytes : (size_t)0);
   float *hbuf = static_cast<float *>(workspace);
   int rc = zt_woq_linear(x, x_dtype, M, K, ldx, w_packed, N, scales, scales_dtype, G, zp,
                          zp_dtype, bias, bias_dtype, nullptr, hbuf, ZT_DT_F32, N,
