@@ -237,6 +237,11 @@ bool s8_prefill_better(int64_t M, int64_t N, int64_t K) {
   const char *e = knob(kKnobS8Kind);
   if (e) return e[0] == 'p';
   const int64_t nk = (K + kPqBK - 1) / kPqBK, tm = (M + 255) / 256;
+  // the load-wave kernel's 256 x 192 tiles where they make one round and its
+  // 256 x 128 do not: 1-3 % ahead up to K = 4096 (quantisation included, M =
+  // 2048: 6144 x 2048 42.4 against 43.3 us, 5120 x 4096 59.7 against 61.1),
+  // behind past it (5120 x 5120 81.0 against 75.3, 6144 x 8192 120.7 against 118)
+  if (tm * ((N + 127) / 128) > 256 && tm * ((N + 191) / 192) <= 256 && K <= 4096) return false;
   return rounds_us(tm * ((N + 255) / 256), nk, 11.0, 1.10, 1.72) <
          rounds_us(tm * ((N + 127) / 128), nk, 8.0, 0.70, 0.98);
 }
