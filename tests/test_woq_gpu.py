@@ -785,3 +785,21 @@ def test_group_modes_gate_up(M, K, I, gs, zp):
     y_ref = O.woq_linear(x, wp[:I].contiguous(), half(s, 0), zero_points=half(z, 0),
                          bias=half(b, 0), post_ops=("silu", "mul"), post_bufs=[up])
     check_close(C.woq_linear_gate_up(*gpu(x, wp, s, z, b)), y_ref)
+
+
+# the stream kernel with two and four tiles per wave in these modes (scales and
+# zero points staged [G][TPW * 16]), ragged N; at 15 rows of 4992 in groups of 64
+# with zero points four tiles would not fit LDS, as at 16 rows in groups of 128
+@pytest.mark.parametrize("M,K,gs,zp,tpw", [
+    (5, 4096, 128, torch.uint8, 2), (5, 4096, 64, None, 2), (5, 4096, 32, torch.int8, 2),
+    (12, 3456, 128, torch.int8, 4), (12, 3456, 64, None, 4), (12, 3456, 32, torch.uint8, 4),
+    (15, 4992, 64, torch.int8, 2), (16, 4992, 128, torch.int8, 2), (16, 4992, 128, None, 2)])
+def test_stream_kernel_tiles_per_wave(M, K, gs, zp, tpw, knobs, capfd):
+    knobs.set("ZT_WOQ_DEBUG", "1")
+    x, wp, s, z, b = group_case(M, K, 12804, gs, zp, M + K + gs)
+    y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b)
+    xd, wd, sd, zd, bd = gpu(x, wp, s, z, b)
+    capfd.readouterr()
+    y = C.woq_linear(xd, wd, sd, zd, bd)
+    assert f"TPW={tpw} " in capfd.readouterr().err
+    check_close(y, y_ref)

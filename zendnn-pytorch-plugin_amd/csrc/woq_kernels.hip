@@ -437,6 +437,12 @@ __host__ __device__ constexpr size_t stream_staged_bytes(int mode, int G, int tp
   return (dec_staged(mode) ? stream_scale_bytes(G, tpw) : 0) +
          (mode == kDecU4G ? stream_zp_bytes(G, tpw) : 0);
 }
+// LDS of a launch: the slabs or x (in p K phases), then what is staged
+inline size_t stream_lds(const WoqArgs &a, int mode, int nw, int tpw, int p, int mt) {
+  const int pitch = p == 1 ? stream_x_pitch((int)a.K) : stream_phase_pitch((int)(a.K / p));
+  return stream_scale_offset(stream_slab_bytes(nw, tpw, mt), (size_t)a.M * pitch * 2) +
+         stream_staged_bytes(mode, (int)a.G, tpw);
+}
 
 // gu > 0 (merged gate_up, fast mode, TPW even, P == MT == 1): weight rows
 // [0, gu) are the gate and [gu, 2 gu) the up projection; tile 2i of the
@@ -1657,11 +1663,7 @@ static hipError_t launch_stream_t(const WoqArgs &a, hipStream_t s, int shift, in
   const int tiles = (int)((a.N + 15) / 16);
   const int x_dma = stream_x_dma(a, P) ? 1 : 0;
   if (P > 1 && !x_dma) return hipErrorInvalidValue;  // phases need the DMA (host-checked)
-  const size_t lds =
-      stream_scale_offset(stream_slab_bytes(NW, TPW, MT),
-                          (size_t)a.M *
-                              (P == 1 ? stream_x_pitch((int)a.K) : stream_phase_pitch((int)(a.K / P))) * 2) +
-      stream_staged_bytes(mode, (int)a.G, TPW);
+  const size_t lds = stream_lds(a, mode, NW, TPW, P, MT);
   dim3 grid((unsigned)((tiles + TPW - 1) / TPW)), block(64 * NW);
   if (mode == kDecFast) {
     woq_stream_kernel<NW, CPW, TPW, kDecFast, P, MT><<<grid, block, lds, s>>>(a, shift, gmask, x_dma, 0);
@@ -1972,13 +1974,7 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
   if (e && e[0] == '0') return false;
   if (e) std::sscanf(e, "%d,%d,%d", &nw, &cpw, &tpw);
   const int mt = (int)((a.M + 15) / 16) == 3 ? 4 : (int)((a.M + 15) / 16);
-  auto fits = [&](int p) {
-    return stream_scale_offset(stream_slab_bytes(nw, tpw, mt),
-                               (size_t)a.M *
-                                   (p == 1 ? stream_x_pitch((int)a.K) : stream_phase_pitch((int)(a.K / p))) * 2) +
-               stream_staged_bytes(mode, (int)a.G, tpw) <=
-           kStreamLdsMax;
-  };
+  auto fits = [&](int p) { return stream_lds(a, mode, nw, tpw, p, mt) <= kStreamLdsMax; };
   // x whole would leave room for one workgroup per CU while the grid makes
   // more than one round: K phases first, whose smaller x range fits two or
   // more workgroups per CU (measured: 10240 x 8192 at M = 6 / 8 took
@@ -2009,8 +2005,9 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
         continue;
       const int cpw_need = p * ((cp + 7) / 8);  // chunks per wave over all phases
       if (knob(kKnobWoqDebug) && !plan_p)
-        std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: MT=%d P=%d CPW>=%d\n",
-                     (long long)a.M, (long long)a.N, (long long)a.K, mt, p, cpw_need);
+        std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: MT=%d P=%d CPW>=%d lds=%zu\n",
+                     (long long)a.M, (long long)a.N, (long long)a.K, mt, p, cpw_need,
+                     stream_lds(a, mode, nw, tpw, p, mt));
 #define ZT_STREAM_PCASE(CPW_, P_, MT_)                                          \
   if (mt == MT_ && p == P_ && cpw_need <= CPW_ && CPW_ % P_ == 0) {            \
     if (plan_p) return *plan_p = P_, true;                                      \
@@ -2037,16 +2034,23 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
   // still leaves most of a round of workgroups (measured: 14336 x 4096 at
   // M = 12 / 16 takes 13.1 / 13.3 us so against 14.0 / 15.1 with two; at
   // M = 8, with two workgroups per CU, four tiles lose)
-  if (!e && (size_t)a.M * stream_x_pitch((int)a.K) * 2 > 76 * 1024 && tiles >= 800 && C <= 64)
+  if (!e && (size_t)a.M * stream_x_pitch((int)a.K) * 2 > 76 * 1024 && tiles >= 800 && C <= 64) {
+    // (twice the slabs and staged scales: 16 x 4992 in groups of 128 would
+    // need 160.6 KB, with zero points in groups of 64 161.2 KB at 15 rows)
+    const int two = tpw;
     tpw = 4;
+    if (!fits(1)) tpw = two;
+  }
+  if (!fits(1)) return false;
   const int need = (C + nw - 1) / nw;
   if (cpw == 0)
     for (int c : {2, 4, 8, 12, 14, 16, 28})
       if (c >= need && ((c != 14 && c != 28) || nw == 8)) { cpw = c; break; }
   if (cpw < need) return false;
   if (knob(kKnobWoqDebug) && !plan_p)
-    std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: NW=%d CPW=%d TPW=%d\n",
-                 (long long)a.M, (long long)a.N, (long long)a.K, nw, cpw, tpw);
+    std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: NW=%d CPW=%d TPW=%d lds=%zu\n",
+                 (long long)a.M, (long long)a.N, (long long)a.K, nw, cpw, tpw,
+                 stream_lds(a, mode, nw, tpw, 1, mt));
 #define ZT_STREAM_CASE(NW_, CPW_, TPW_) \
   if (nw == NW_ && cpw == CPW_ && tpw == TPW_) { \
     if (plan_p) return *plan_p = 1, true; \
@@ -2700,8 +2704,7 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
     WidePlan wp;
     if (woq_wide_ok(a, &wp) && wp.splits == 1) return false;
   }
-  const size_t lds = stream_scale_offset(stream_slab_bytes(8, tpw, 1), x_bytes) +
-                     stream_staged_bytes(mode, (int)a.G, tpw);
+  const size_t lds = stream_lds(a, mode, 8, tpw, 1, 1);
   if (lds > kStreamLdsMax) return false;
   const int need = (C + 7) / 8;
   int cpw = 0;
@@ -2711,8 +2714,8 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   const int x_dma = stream_x_dma(a, 1) ? 1 : 0;
   const dim3 grid((unsigned)((I / 16 + tpw / 2 - 1) / (tpw / 2))), block(512);
   if (knob(kKnobWoqDebug))
-    std::fprintf(stderr, "[zt] woq gate_up stream M=%lld N=%lld K=%lld: CPW=%d TPW=%d\n",
-                 (long long)a.M, (long long)a.N, (long long)a.K, cpw, tpw);
+    std::fprintf(stderr, "[zt] woq gate_up stream M=%lld N=%lld K=%lld: CPW=%d TPW=%d lds=%zu\n",
+                 (long long)a.M, (long long)a.N, (long long)a.K, cpw, tpw, lds);
 #define ZT_GU_MODE(CPW_, TPW_, MODE_)                                                       \
   woq_stream_kernel<8, CPW_, TPW_, MODE_, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask,  \
                                                                         x_dma, (int)I)
