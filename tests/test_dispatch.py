@@ -22,3 +22,13 @@ def test_stream_launches_fit_lds():
                 seen += 1
                 assert int(m.group(1)) <= LDS, (call, line)
     assert seen > len(calls) // 2
+
+
+# a forced layout of other than eight waves is the general mode's: 8-bit zero
+# points and groups of 64 leave the stream kernel's modes for it and still run
+def test_forced_stream_layout_of_other_waves():
+    calls = [dict(M=8, K=1024, N=64, zp="int8"), dict(M=8, K=1024, N=64, zp="uint8", gs=256),
+             dict(M=8, K=1024, N=64, gs=64), dict(M=8, K=1024, N=64, gs=64, gate_up=True)]
+    for status, lines in plans(calls, ZT_WOQ_STREAM="4,2,1"):
+        assert "invalid argument" not in status, (status, lines)
+        assert lines

@@ -1973,6 +1973,9 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
   const char *e = knob(kKnobWoqStream);  // "0" disables; "NW,CPW,TPW" forces
   if (e && e[0] == '0') return false;
   if (e) std::sscanf(e, "%d,%d,%d", &nw, &cpw, &tpw);
+  // (the group modes are built for eight waves: other forced layouts are left
+  // to the general mode)
+  if ((mode == kDecS4G || mode == kDecU4G) && nw != 8) return false;
   const int mt = (int)((a.M + 15) / 16) == 3 ? 4 : (int)((a.M + 15) / 16);
   auto fits = [&](int p) { return stream_lds(a, mode, nw, tpw, p, mt) <= kStreamLdsMax; };
   // x whole would leave room for one workgroup per CU while the grid makes
