@@ -803,3 +803,28 @@ def test_stream_kernel_tiles_per_wave(M, K, gs, zp, tpw, knobs, capfd):
     y = C.woq_linear(xd, wd, sd, zd, bd)
     assert f"TPW={tpw} " in capfd.readouterr().err
     check_close(y, y_ref)
+
+
+# 8-bit zero points with scales near the end of the fp32 range and infinite
+# ones: the weights are (u - z) * s, finite and infinite alike, on every kernel.
+# (u - z keeps one sign, so that infinite products do not meet their negatives.)
+@pytest.mark.parametrize("M,N,force", [(4, 64, None), (24, 132, "wide"), (40, 132, "wide"),
+                                       (130, 64, "gemm")])
+@pytest.mark.parametrize("big", [3e35, -1e36, float("inf"), float("-inf"), 1e-36])
+@pytest.mark.parametrize("zp,z0", [(torch.int8, -1), (torch.uint8, 200), (torch.int8, -128)])
+@pytest.mark.parametrize("gs", [128, 32])
+def test_zero_points_scale_range(M, N, force, big, zp, z0, gs, knobs):
+    K = 256
+    g = torch.Generator().manual_seed(M + N)
+    u = torch.randint(0, 16, (N, K), generator=g, dtype=torch.int8)
+    s = torch.full((K // gs, N), 0.01)
+    s[0, ::2] = big
+    s = s.bfloat16()
+    z = torch.full((K // gs, N), z0).to(zp)
+    x = (torch.rand(M, K, generator=g) * 2 ** -10 + 2 ** -10).bfloat16()
+    w = (u.float() - z.float().t().repeat_interleave(gs, 1)) * s.float().t().repeat_interleave(gs, 1)
+    y_ref = x.double() @ w.bfloat16().double().t()
+    knobs.set("ZT_WOQ_FORCE_KERNEL", force)
+    y = C.woq_linear(*gpu(x, O.woq_repack_weight(u), s, z))
+    # (bf16 outputs: 2^-9, and fp32 sums of 256 terms of one sign)
+    torch.testing.assert_close(y.cpu().double(), y_ref, rtol=2 ** -8, atol=0)

@@ -59,12 +59,46 @@ __device__ __forceinline__ u32x4_t dq8_s4_bf16scale(uint32_t w, float s, float s
   return r;
 }
 
-// Unsigned int4 with a bf16 scale s and an 8-bit integer zero point z:
+// Unsigned int4 with a scale s and an 8-bit integer zero point z: the exact
+// integers u - z two at a time in fp16,
+//   (1024 + u) - (1024 + z)        v_pk_add_f16
+//   (1024 + 16u) / 16 - (64 + z)   v_pk_fma_f16
+// (1024 + z, 64 + z and u - z are integers below 2048), then their fp32
+// product with s, the reference's own arithmetic: with the zero point folded
+// into one fma, -(1024 + z) s, a scale past 2.6e35 overflowed where (u - z) s
+// does not, and an infinite one made every weight a NaN.
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4_t dq8_u4_scale(uint32_t w, float s, float z) {
+  const uint32_t w8 = w >> 8;
+  const _Float16 o0 = (_Float16)(-1024.f - z), o1 = (_Float16)(-64.f - z), r16 = (_Float16)0.0625f;
+  auto lo = [&](uint32_t t) {
+    return __builtin_bit_cast(f16x2_t, and_xor(t, kNibLo, kExpLo)) + f16x2_t{o0, o0};
+  };
+  auto hi = [&](uint32_t t) {
+    return __builtin_elementwise_fma(__builtin_bit_cast(f16x2_t, and_xor(t, kNibHi, kExpLo)),
+                                     f16x2_t{r16, r16}, f16x2_t{o1, o1});
+  };
+  // t * s + -0 is t * s, and one v_fma_mix_f32 where t * s is a conversion and a
+  // multiplication; the compiler may not see that the addend is -0
+  float none = -0.f;
+  asm("" : "+s"(none));
+  auto mul = [&](_Float16 t) { return fmaf((float)t, s, none); };
+  const f16x2_t q0 = lo(w), q1 = hi(w), q2 = lo(w8), q3 = hi(w8);
+  u32x4_t r;
+  r[0] = pack_bf16x2(mul(q0[0]), mul(q1[0]));
+  r[1] = pack_bf16x2(mul(q2[0]), mul(q3[0]));
+  r[2] = pack_bf16x2(mul(q0[1]), mul(q1[1]));
+  r[3] = pack_bf16x2(mul(q2[1]), mul(q3[1]));
+  return r;
+}
+
+// The same for |s| < kSmallScale with the zero point folded into one fma,
 //   fma(1024 + u,   s,    -(1024 + z) s) = (u - z) s
-//   fma(1024 + 16u, s/16, -(64 + z) s)   = (u - z) s
-// exact as above: 1024 + z and 64 + z have at most 11 significant bits, so
-// their products with s at most 19, and (u - z) s at most 17.
-__device__ __forceinline__ u32x4_t dq8_u4_bf16scale(uint32_t w, float s, float z) {
+//   fma(1024 + 16u, s/16, -(64 + z) s)   = (u - z) s,
+// exact for bf16 scales: 1024 + z and 64 + z have at most 11 significant
+// bits, so their products with s at most 19, and (u - z) s at most 17.
+constexpr float kSmallScale = 0x1p117f;  // 1279 * 2^117 < 2^128
+__device__ __forceinline__ u32x4_t dq8_u4_small_scale(uint32_t w, float s, float z) {
   const uint32_t w8 = w >> 8;
   const uint32_t p0 = and_xor(w, kNibLo, kExpLo);
   const uint32_t p1 = and_xor(w, kNibHi, kExpLo);

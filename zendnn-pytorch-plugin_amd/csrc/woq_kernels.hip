@@ -125,8 +125,11 @@ constexpr unsigned kCounterSlots = 1024;  // 4096-byte counter region
 // in groups of 128 and up (the fast path); the general path with bf16 / fp32
 // scales; and, on the stream and wide kernels, bf16 scales in groups of 32
 // and up (a lane of the decode layout holds exactly one block of 32), signed
-// or with 8-bit zero points, at the fast path's one FMA per weight.
-enum DecodeMode { kDecFast = 0, kDecGenBf16 = 1, kDecGenF32 = 2, kDecS4G = 3, kDecU4G = 4 };
+// or with 8-bit zero points.  kDecU4Small is kDecU4G on scales below
+// kSmallScale, at the fast path's one FMA per weight.
+enum DecodeMode {
+  kDecFast = 0, kDecGenBf16 = 1, kDecGenF32 = 2, kDecS4G = 3, kDecU4G = 4, kDecU4Small = 5
+};
 
 // Modes whose scales (and zero points) the stream kernel stages in LDS.
 __host__ __device__ constexpr bool dec_staged(int mode) {
@@ -145,7 +148,9 @@ __device__ __forceinline__ bf16x8_t dq_word(uint32_t w, float s, float z, int zm
   if (MODE == kDecFast || MODE == kDecS4G)
     v = dq8_s4_bf16scale(w, s, s * 0.0625f, -1032.f * s, -72.f * s);
   else if (MODE == kDecU4G)
-    v = dq8_u4_bf16scale(w, s, z);
+    v = dq8_u4_scale(w, s, z);
+  else if (MODE == kDecU4Small)
+    v = dq8_u4_small_scale(w, s, z);
   else
     v = dq8_general(w, dq_general_params(zmode, s, z));
   return __builtin_bit_cast(bf16x8_t, v);
@@ -607,6 +612,8 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
     if (kc < C) {
       const int kcl = P == 1 ? kc : kc - (c / CPWP) * CP;  // chunk within the LDS range
       bf16x8_t wb[TPW][4];
+      float su[TPW], zu[TPW];
+      bool large = false;  // kDecU4G: a scale past kDecU4Small's range
 #pragma unroll
       for (int t = 0; t < TPW; ++t) {
         // the lane's scale group: cpg_shift counts chunks in the fast mode,
@@ -618,7 +625,18 @@ __global__ __launch_bounds__(64 * NW) void woq_stream_kernel(WoqArgs a, int cpg_
         const float sc = MODE == kDecGenF32 ? __uint_as_float(sb) : __uint_as_float(sb << 16);
         const float zc = MODE == kDecU4G ? (float)(((int)zl[at] ^ zsx) - zsx) : zr[t][c];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) wb[t][i] = dq_word<MODE>(wr[t][c][i], sc, zc, zmode);
+        for (int i = 0; i < 4; ++i)
+          wb[t][i] = dq_word<MODE == kDecU4G ? kDecU4Small : MODE>(wr[t][c][i], sc, zc, zmode);
+        su[t] = sc, zu[t] = zc;
+        large = large || !(fabsf(sc) < kSmallScale);
+      }
+      // (kDecU4G on every chunk took 5-11 % more at 1 to 8 rows: 18944 x 3584 at
+      // M = 8 15.6 us against 14.2, 28672 x 4096 at M = 1 17.3 against 15.9)
+      if (MODE == kDecU4G && __builtin_expect(__builtin_amdgcn_ballot_w64(large) != 0, 0)) {
+#pragma unroll
+        for (int t = 0; t < TPW; ++t)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) wb[t][i] = dq_word<kDecU4G>(wr[t][c][i], su[t], zu[t], 0);
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {

@@ -12,9 +12,9 @@ namespace zt {
 
 namespace {
 
-// How the workgroup dequantises: signed int4 with bf16 scales, unsigned
-// int4 with bf16 scales and 8-bit integer zero points (both one FMA per
-// weight), or any scale / zero-point type.
+// How the workgroup dequantises: signed int4 with bf16 scales (one FMA per
+// weight), unsigned int4 with bf16 scales and 8-bit integer zero points (and
+// half a packed fp16 one), or any scale / zero-point type.
 enum DequantMode { kDqS4 = 0, kDqU4 = 1, kDqAny = 2 };
 
 // Cost model of woq_prefill_plan, microseconds: a tile's prologue and
@@ -99,7 +99,7 @@ __device__ __forceinline__ GroupQ group_of(const GroupFormat &f, GroupRaw r) {
 template <int DQ>
 __device__ __forceinline__ u32x4_t dequant8(uint32_t w, const GroupQ &q, int zmode) {
   if (DQ == kDqS4) return dq8_s4_bf16scale(w, q.s, q.s * 0.0625f, -1032.f * q.s, -72.f * q.s);
-  if (DQ == kDqU4) return dq8_u4_bf16scale(w, q.s, q.z);
+  if (DQ == kDqU4) return dq8_u4_scale(w, q.s, q.z);
   return dq8_general(w, dq_general_params(zmode, q.s, q.z));
 }
 
