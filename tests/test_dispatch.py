@@ -32,3 +32,18 @@ def test_forced_stream_layout_of_other_waves():
     for status, lines in plans(calls, ZT_WOQ_STREAM="4,2,1"):
         assert "invalid argument" not in status, (status, lines)
         assert lines
+
+
+# 17..64 rows with fp32 scales, or zero points that the wide kernel does not
+# take: blocks of 16 rows on small matrices and few rows, the large-tile
+# kernel where it reads the weights once for more
+def test_general_modes_17_to_64_rows():
+    cases = [(dict(M=M, K=K, N=N, **kind), prefill)
+             for kind in (dict(s_dtype="float32"), dict(zp="bfloat16"), dict(zp="int32"))
+             for M, K, N, prefill in [
+                 (17, 4096, 4096, False), (32, 2048, 2048, False), (24, 4096, 512, False),
+                 (32, 256, 256, False), (24, 2048, 1001, False), (33, 4096, 4096, False),
+                 (64, 4096, 4096, True), (48, 4096, 14336, True), (24, 3584, 18944, True),
+                 (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 256, 256, True)]]
+    for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert lines and lines[0].startswith("woq prefill") == prefill, (call, lines)

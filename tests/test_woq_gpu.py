@@ -736,14 +736,15 @@ def test_prefill_kernel_gate_up(M, K, I, gs, zp, tile, knobs):
     run_gate_up(M, K, I, K // gs, seed=M + I, zp=zp)
 
 
-# zero points at 17..64 rows: the prefill kernel when the workspace holds its
-# splits
-@pytest.mark.parametrize("M,K,N", [(17, 4096, 520), (64, 2048, 261)])
-def test_zero_points_17_to_64_rows(M, K, N, knobs, capfd):
+# 32-bit zero points at 17..64 rows: the prefill kernel, K split over the
+# workspace, where it beats blocks of 16 rows (test_dispatch.py has the line)
+@pytest.mark.parametrize("M,K,N,prefill", [(17, 4096, 520, False), (17, 14336, 520, True),
+                                           (64, 2048, 261, True)])
+def test_zero_points_17_to_64_rows(M, K, N, prefill, knobs, capfd):
     knobs.set("ZT_WOQ_DEBUG", "1")
     capfd.readouterr()
     run_case(M, K, N, K // 128, zp="int", seed=M + N, bias=True)
-    assert "woq prefill" in capfd.readouterr().err
+    assert ("woq prefill" in capfd.readouterr().err) == prefill
 
 
 # 8-bit zero points and groups of 32 / 64 on the decode kernels: the stream

@@ -358,13 +358,12 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   // 17..64 rows with fp32 scales or zero points the wide kernel does not
   // take: the prefill GEMM, K split over the workspace, reads the weights
   // once where the decode kernels' general modes pay their longer
-  // dequantisation per row block (zero points, 24 / 64 rows: 4096 x 4096 17.8 /
-  // 34.6 -> 16.8 / 21.2 us, 18944 x 3584 68.7 / 167 -> 31.0 / 35.1,
-  // 3584 x 18944 62.4 / 131 -> 33.5 / 37.1)
+  // dequantisation per row block
   if (M > kWoqRowBlock && M <= kWoqRowBlockMax && (zp || scales_dtype == ZT_DT_F32) &&
       !zt::knob(zt::kKnobWoqForceKernel) && !zt::knob(zt::kKnobWoqStream) &&
-      zt::woq_prefill_ok(a) && workspace &&
-      workspace_bytes >= zt::woq_prefill_workspace(M, N, K))
+      zt::woq_prefill_ok(a) &&
+      zt::woq_prefill_workspace(M, N, K) <= (workspace ? workspace_bytes : 0) &&
+      (!woq_use_row_blocks(a) || zt::woq_prefill_beats_row_blocks(a)))
     return hip_status(zt::launch_woq_prefill(a, false, workspace, workspace_bytes, s), op);
   if (woq_use_row_blocks(a)) {
     // one stream-kernel launch over all rows when x (in K phases) fits, else

@@ -1,5 +1,6 @@
 // Large-tile int4 weight-only GEMM for gfx950 (prefill, any zero-point and
 // scale type, groups of 32 and up).
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -486,6 +487,30 @@ PrefillPlan woq_prefill_plan(int64_t M, int64_t N, int64_t K, bool gate_up) {
     }
   }
   return best;
+}
+
+// Both sides from graph replays at 17 to 64 rows of 28 shapes, 256 x 256 to
+// 28672 x 4096 (bf16 zero points; fp32 scales; 8-bit zero points where N % 4
+// keeps the wide kernel away).  The choice is the faster one, or within 2 %, at
+// 422 of 427 points; 17 x 4096 x 4096 took 22.3 / 23.6 us (zero points / fp32
+// scales) here against 14.4 / 13.0 in blocks, 64 x 4096 x 4096 24 / 25 against 31 /
+// 28, 24 x 18944 x 3584 35 / 40 against 70 / 54.
+bool woq_prefill_beats_row_blocks(const WoqArgs &a) {
+  const double plan = woq_prefill_plan(a.M, a.N, a.K, false).us;
+  const bool f32 = a.s_dt == ZT_DT_F32;
+  // (the plan's constants are those of the two one-FMA dequantisations)
+  const double here = f32                                               ? 1.32 * plan + 0.7
+                      : a.zp_dt == ZT_DT_S8 || a.zp_dt == ZT_DT_U8 ? 0.9 * plan
+                                                                        : 1.13 * plan + 1.6;
+  // a round of 256 row tiles of 16, x whole in LDS (stream kernel) or not
+  const double k = (double)a.K;
+  const double round =
+      16 * (a.K + 8) * 2 <= 160 * 1024
+          ? std::min(0.7 + 0.0035 * k, f32 ? 2.7 + 0.00045 * k : 2.5 + 0.0007 * k)
+          : (f32 ? 0.0014 : 0.0016) * k;
+  const int64_t rounds = ((a.N + 15) / 16 + 255) / 256, blocks = (a.M + 15) / 16;
+  const double last = 0.6 + 0.4 / 16 * (double)(a.M - 16 * (blocks - 1));
+  return here < (3.0 + rounds * round) * (blocks - 1 + last);
 }
 
 size_t woq_prefill_workspace(int64_t M, int64_t N, int64_t K) {

@@ -68,6 +68,10 @@ struct PrefillPlan {
 bool woq_prefill_ok(const WoqArgs &a);
 PrefillPlan woq_prefill_plan(int64_t M, int64_t N, int64_t K, bool gate_up);
 size_t woq_prefill_workspace(int64_t M, int64_t N, int64_t K);
+// 17..64 rows with zero points or fp32 scales: whether the kernel above, with
+// room for its splits, is estimated faster than blocks of 16 rows on the decode
+// kernels' general modes.
+bool woq_prefill_beats_row_blocks(const WoqArgs &a);
 hipError_t launch_woq_prefill(const WoqArgs &a, bool gate_up, void *workspace,
                               size_t workspace_bytes, hipStream_t s);
 int woq_gemm_splits(int64_t M, int64_t N, int64_t K);
