@@ -47,3 +47,23 @@ def test_general_modes_17_to_64_rows():
                  (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 256, 256, True)]]
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert lines and lines[0].startswith("woq prefill") == prefill, (call, lines)
+
+
+# merged gate_up on the large tiles: in one launch where its tiles fill the GPU
+# or the workspace holds no K split of the plain linear, else in two steps
+def test_gate_up_large_tiles_or_two_steps():
+    general = (dict(s_dtype="float32"), dict(zp="bfloat16"))
+    cases = [(dict(M=M, K=K, N=N, gate_up=True, **kind), merged)
+             for kind in (dict(), dict(gs=32), dict(zp="int8")) + general
+             for M, K, N, merged in [
+                 (128, 4096, 28672, True), (512, 4096, 7168, True), (2048, 14336, 8192, True),
+                 (300, 512, 512, True), (128, 4096, 3584, False), (128, 14336, 1024, False),
+                 (200, 8192, 7168, False), (1024, 14336, 1024, False)]]
+    cases += [(dict(M=M, K=K, N=N, gate_up=True, **kind), False)
+              for kind in general for M, K, N in [(17, 4096, 3584), (32, 14336, 1024),
+                                                  (64, 2048, 2048), (24, 512, 512)]]
+    cases += [(dict(M=128, K=4096, N=3584, gate_up=True, workspace=4 * 128 * 3584), True),
+              (dict(M=64, K=4096, N=28672, gate_up=True, zp="bfloat16"), False),
+              (dict(M=64, K=3584, N=37888, gate_up=True, zp="bfloat16"), True)]
+    for (call, merged), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert any(l.endswith(", gate_up") for l in lines) == merged, (call, lines)

@@ -437,11 +437,24 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   // would take that kernel too; the decode kernels keep the two steps
   const char *forced = zt::knob(zt::kKnobWoqGemm);
   zt::WidePlan wp;
+  const bool general = zp || scales_dtype == ZT_DT_F32;
   const bool decode = M <= kWoqRowBlockMax && !(forced && forced[0] == 'p') &&
                       (zt::woq_wide_ok(a, &wp) || zt::woq_group_stream_ok(a) ||
-                       (M > kWoqRowBlock ? !zp && scales_dtype != ZT_DT_F32 && woq_use_row_blocks(a)
+                       (M > kWoqRowBlock ? woq_use_row_blocks(a) &&
+                                               !(general && zt::woq_prefill_ok(a) &&
+                                                 zt::woq_prefill_beats_row_blocks(a))
                                          : zt::woq_select_kernel(a) == zt::kWoqDecode));
-  if (!decode && (!forced || forced[0] == 'p') && zt::woq_prefill_ok(a))
+  // Few tiles: the plain linear splits K where the merged form, whose sums
+  // meet only in its epilogue, cannot.  The two steps are taken where the
+  // split's estimate is the lower one (the silu * up pass weighs as much as the
+  // estimate is too high by): the faster side, or within 12 %, at all of 1282
+  // points of 19 shapes at 17 to 2048 rows (1024 x 14336 at M = 128 31 us against
+  // 143 merged, 3584 x 4096 24 against 41; 28672 x 4096 merged 47 against 53).
+  const size_t split = zt::woq_prefill_workspace(M, N, K);
+  const bool two_steps = split && split <= workspace_bytes - h && !forced &&
+                         zt::woq_prefill_plan(M, N, K, false).us <
+                             zt::woq_prefill_plan(M, N, K, true).us;
+  if (!decode && !two_steps && (!forced || forced[0] == 'p') && zt::woq_prefill_ok(a))
     return hip_status(zt::launch_woq_prefill(a, true, nullptr, 0, s), op);
   // two steps: the full [M, N] linear in fp32 into the workspace, then
   // silu(gate) * up over its halves
