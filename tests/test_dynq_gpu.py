@@ -411,3 +411,22 @@ def test_s8_256_tile_kernel(kind, M, N, K, knobs):
                                  out_dtype=torch.int32).cpu()
     q, _, zp = O.dynamic_quantize_asym(x)
     assert torch.equal(acc, (q.int() - zp[:, None].int()) @ w.t().int())
+
+
+# fp32 and bf16 binary operands of other row strides than N in the tile
+# epilogues: the 256 x 256 kernel, the load-wave kernel and its other tiles
+@pytest.mark.parametrize("kind,tile", [("p", None), ("w", None), ("w", "1"), ("w", "9")])
+@pytest.mark.parametrize("op_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("ld", [264, 272, 267])
+def test_s8_strided_operands(kind, tile, op_dtype, ld, knobs):
+    M, N, K = 300, 264, 384
+    knobs.set("ZT_S8_KIND", kind)
+    knobs.set("ZT_S8_TILE", tile)
+    x, w, sw, b = make(M, K, N, seed=ld, x_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(ld)
+    bufs = [torch.randn(M, ld, generator=g).to(op_dtype) for _ in range(2)]
+    y_ref = O.dynamic_qlinear(x, w, sw, b, post_ops=("mul", "add"),
+                              post_bufs=[t[:, :N].contiguous() for t in bufs])
+    y = C.dynamic_qlinear(x.to(DEV), w.to(DEV), sw.to(DEV), b.to(DEV), post_ops=("mul", "add"),
+                          post_bufs=[t.to(DEV)[:, :N] for t in bufs]).cpu()
+    torch.testing.assert_close(y.float(), y_ref.float(), rtol=1e-2, atol=1e-2)

@@ -829,3 +829,31 @@ def test_zero_points_scale_range(M, N, force, big, zp, z0, gs, knobs):
     y = C.woq_linear(*gpu(x, O.woq_repack_weight(u), s, z))
     # (bf16 outputs: 2^-9, and fp32 sums of 256 terms of one sign)
     torch.testing.assert_close(y.cpu().double(), y_ref, rtol=2 ** -8, atol=0)
+
+
+# x and binary post-op operands with rows longer than K and N on the large tiles
+# (every tile, and the load-wave kernel): fp32 and bf16 operands whose rows are
+# and are not whole 16- or 8-byte pieces, ragged M and N
+@pytest.mark.parametrize("variant", ["p01", "p11", "p21", "p03", "v"])
+@pytest.mark.parametrize("op_dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("M,N,ld", [(130, 264, 264), (300, 264, 272), (130, 264, 267)])
+def test_prefill_strided_operands(variant, op_dtype, M, N, ld, knobs):
+    K, G = 1024, 8
+    knobs.set("ZT_WOQ_FORCE_KERNEL", "gemm")
+    knobs.set("ZT_WOQ_GEMM", variant)
+    x, q, wp, s, z, b = make_case(M, K + 24, N, 1, seed=M + ld, bias=True)
+    x, q = x[:, :K], q[:, :K].contiguous()
+    wp, s = O.woq_repack_weight(q), torch.rand(G, N).mul(0.015).add(0.005).bfloat16()
+    g = torch.Generator().manual_seed(ld)
+    bufs = [torch.randn(M, ld, generator=g).to(op_dtype)[:, :N] for _ in range(2)]
+    y_ref = O.woq_linear(x.contiguous(), wp, s, bias=b, post_ops=("mul", "add"),
+                         post_bufs=[t.contiguous() for t in bufs])
+    xd, wd, sd, bd = gpu(x, wp, s, b)
+    big = [torch.zeros(M, ld, dtype=op_dtype, device=DEV) for _ in bufs]
+    for d, t in zip(big, bufs):
+        d[:, :N] = t.to(DEV)
+    xs = torch.zeros(M, K + 24, dtype=x.dtype, device=DEV)
+    xs[:, :K] = xd
+    y = C.woq_linear(xs[:, :K], wd, sd, None, bd, post_ops=("mul", "add"),
+                     post_bufs=[d[:, :N] for d in big])
+    check_close(y, y_ref)

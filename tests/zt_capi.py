@@ -121,11 +121,12 @@ def make_post(post_ops, bufs, N):
     for i, name in enumerate(post_ops):
         po.ids[i] = PO[name]
         if name in ("add", "mul"):
-            b = bufs[bi].reshape(-1, N).contiguous()
+            b = bufs[bi].reshape(-1, N)  # rows of any stride
+            b = b if b.stride(1) == 1 else b.contiguous()
             keep.append(b)
             po.bufs[bi] = b.data_ptr()
             po.buf_dtypes[bi] = DT[b.dtype]
-            po.buf_ld[bi] = N
+            po.buf_ld[bi] = b.stride(0) if b.shape[0] > 1 else N
             bi += 1
     return po, keep
 

@@ -118,19 +118,32 @@ __device__ __forceinline__ void post_ops_slab(float *slab, int pitch, int c4, in
       const int es = f32 ? 4 : 2;
       const char *base = static_cast<const char *>(p.bufs[b]) + (int64_t)n * es;
       const int64_t ld = p.ld[b] * es;
-      const bool vec = n + 3 < N && !f32 && ((reinterpret_cast<uintptr_t>(base) | ld) & 7) == 0;
-      if (vec) {
+      const bool vec =
+          n + 3 < N && ((reinterpret_cast<uintptr_t>(base) | ld) & (f32 ? 15 : 7)) == 0;
+      auto row = [&](int t) { return base + min(mb + t * RP + r0, M - 1) * ld; };
+      auto apply = [&](int t, f32x4_t w) {
+        f32x4_t *q = reinterpret_cast<f32x4_t *>(slab + (t * RP + r0) * pitch + c4);
+        *q = id == ZT_PO_ADD ? *q + w : *q * w;
+      };
+      if (vec && f32) {
+        constexpr int U = T < 8 ? T : 8;  // rows in flight
+        static_assert(T % U == 0, "whole batches");
+#pragma unroll 1
+        for (int t0 = 0; t0 < T; t0 += U) {
+          f32x4_t o[U];
+#pragma unroll
+          for (int t = 0; t < U; ++t) o[t] = *reinterpret_cast<const f32x4_t *>(row(t0 + t));
+#pragma unroll
+          for (int t = 0; t < U; ++t) apply(t0 + t, o[t]);
+        }
+      } else if (vec) {
         u32x2_t o[T];
 #pragma unroll
-        for (int t = 0; t < T; ++t)
-          o[t] = *reinterpret_cast<const u32x2_t *>(base + min(mb + t * RP + r0, M - 1) * ld);
+        for (int t = 0; t < T; ++t) o[t] = *reinterpret_cast<const u32x2_t *>(row(t));
 #pragma unroll
-        for (int t = 0; t < T; ++t) {
-          f32x4_t *q = reinterpret_cast<f32x4_t *>(slab + (t * RP + r0) * pitch + c4);
-          const f32x4_t w = {bf16_bits_to_f32(o[t][0] & 0xffffu), __uint_as_float(o[t][0] & 0xffff0000u),
-                             bf16_bits_to_f32(o[t][1] & 0xffffu), __uint_as_float(o[t][1] & 0xffff0000u)};
-          *q = id == ZT_PO_ADD ? *q + w : *q * w;
-        }
+        for (int t = 0; t < T; ++t)
+          apply(t, f32x4_t{bf16_bits_to_f32(o[t][0] & 0xffffu), __uint_as_float(o[t][0] & 0xffff0000u),
+                           bf16_bits_to_f32(o[t][1] & 0xffffu), __uint_as_float(o[t][1] & 0xffff0000u)});
       } else {
 #pragma unroll 1
         for (int t = 0; t < T; ++t) {
