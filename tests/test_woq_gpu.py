@@ -755,16 +755,18 @@ def group_case(M, K, N, gs, zp, seed):
     return x, wp, s, z.to(zp) if zp else None, b
 
 
-@pytest.mark.parametrize("M,K,N,kernel", [
-    (1, 1024, 40, "stream"), (4, 3584, 132, "stream"), (16, 4096, 260, "stream"),
+GROUP_CASES = [
+    (1, 2176, 40, "stream"), (4, 3584, 132, "stream"), (16, 4096, 260, "stream"),
     (9, 14336, 68, "stream"), (3, 2176, 36, "stream"), (30, 4096, 260, "stream"),
     (64, 2048, 132, "stream"), (17, 11008, 1540, "wide"), (33, 3584, 4164, "wide"),
-    (64, 1280, 4164, "wide"), (12, 13824, 5124, "wide"), (17, 11008, 136, "prefill")])
-@pytest.mark.parametrize("gs,zp", [(128, torch.int8), (64, torch.uint8), (64, None),
-                                   (32, torch.int8), (32, None), (256, torch.uint8)])
+    (64, 1280, 4164, "wide"), (12, 13824, 5124, "wide"), (17, 11008, 136, "prefill")]
+GROUP_MODES = [(128, torch.int8), (64, torch.uint8), (64, None), (32, torch.int8), (32, None),
+               (256, torch.uint8)]
+
+
+@pytest.mark.parametrize("M,K,N,kernel,gs,zp", [c + m for m in GROUP_MODES for c in GROUP_CASES
+                                                if c[1] % m[0] == 0])
 def test_group_modes_decode(M, K, N, kernel, gs, zp, knobs, capfd):
-    if K % gs or (K // gs * gs != K):
-        pytest.skip("K is not whole groups")
     knobs.set("ZT_WOQ_DEBUG", "1")
     x, wp, s, z, b = group_case(M, K, N, gs, zp, M + K + N + gs)
     y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b, post_ops=("relu",))

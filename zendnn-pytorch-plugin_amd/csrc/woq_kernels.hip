@@ -2025,13 +2025,14 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
           fits(4) && half_x(4) && 4 * ((C / 4 + 7) / 8) <= 28)
         continue;
       const int cpw_need = p * ((cp + 7) / 8);  // chunks per wave over all phases
-      if (knob(kKnobWoqDebug) && !plan_p)
-        std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: MT=%d P=%d CPW>=%d lds=%zu\n",
-                     (long long)a.M, (long long)a.N, (long long)a.K, mt, p, cpw_need,
-                     stream_lds(a, mode, nw, tpw, p, mt));
 #define ZT_STREAM_PCASE(CPW_, P_, MT_)                                          \
   if (mt == MT_ && p == P_ && cpw_need <= CPW_ && CPW_ % P_ == 0) {            \
     if (plan_p) return *plan_p = P_, true;                                      \
+    if (knob(kKnobWoqDebug))                                                    \
+      std::fprintf(stderr,                                                      \
+                   "[zt] woq stream M=%lld N=%lld K=%lld: MT=%d P=%d CPW=%d lds=%zu\n", \
+                   (long long)a.M, (long long)a.N, (long long)a.K, mt, p, CPW_, \
+                   stream_lds(a, mode, nw, tpw, p, mt));                        \
     *err = launch_stream_t<8, CPW_, 1, P_, MT_>(a, s, shift, gmask, mode);      \
     return true;                                                                \
   }
@@ -2068,13 +2069,13 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
     for (int c : {2, 4, 8, 12, 14, 16, 28})
       if (c >= need && ((c != 14 && c != 28) || nw == 8)) { cpw = c; break; }
   if (cpw < need) return false;
-  if (knob(kKnobWoqDebug) && !plan_p)
-    std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: NW=%d CPW=%d TPW=%d lds=%zu\n",
-                 (long long)a.M, (long long)a.N, (long long)a.K, nw, cpw, tpw,
-                 stream_lds(a, mode, nw, tpw, 1, mt));
 #define ZT_STREAM_CASE(NW_, CPW_, TPW_) \
   if (nw == NW_ && cpw == CPW_ && tpw == TPW_) { \
     if (plan_p) return *plan_p = 1, true; \
+    if (knob(kKnobWoqDebug)) \
+      std::fprintf(stderr, "[zt] woq stream M=%lld N=%lld K=%lld: NW=%d CPW=%d TPW=%d lds=%zu\n", \
+                   (long long)a.M, (long long)a.N, (long long)a.K, nw, cpw, tpw, \
+                   stream_lds(a, mode, nw, tpw, 1, mt)); \
     *err = launch_stream_t<NW_, CPW_, TPW_>(a, s, shift, gmask, mode); return true; }
   ZT_STREAM_CASE(4, 2, 1) ZT_STREAM_CASE(4, 4, 1) ZT_STREAM_CASE(4, 8, 1) ZT_STREAM_CASE(4, 12, 1)
   ZT_STREAM_CASE(4, 16, 1) ZT_STREAM_CASE(4, 8, 2) ZT_STREAM_CASE(4, 4, 2) ZT_STREAM_CASE(4, 16, 2)
@@ -2734,14 +2735,15 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   if (cpw < need) return false;
   const int x_dma = stream_x_dma(a, 1) ? 1 : 0;
   const dim3 grid((unsigned)((I / 16 + tpw / 2 - 1) / (tpw / 2))), block(512);
-  if (knob(kKnobWoqDebug))
-    std::fprintf(stderr, "[zt] woq gate_up stream M=%lld N=%lld K=%lld: CPW=%d TPW=%d lds=%zu\n",
-                 (long long)a.M, (long long)a.N, (long long)a.K, cpw, tpw, lds);
 #define ZT_GU_MODE(CPW_, TPW_, MODE_)                                                       \
   woq_stream_kernel<8, CPW_, TPW_, MODE_, 1, 1><<<grid, block, lds, s>>>(a, shift, gmask,  \
                                                                         x_dma, (int)I)
 #define ZT_GU_CASE(CPW_, TPW_)                                                              \
   if (cpw == CPW_ && tpw == TPW_) {                                                        \
+    if (knob(kKnobWoqDebug))                                                               \
+      std::fprintf(stderr,                                                                 \
+                   "[zt] woq gate_up stream M=%lld N=%lld K=%lld: CPW=%d TPW=%d lds=%zu\n", \
+                   (long long)a.M, (long long)a.N, (long long)a.K, cpw, tpw, lds);         \
     if (mode == kDecFast) ZT_GU_MODE(CPW_, TPW_, kDecFast);                                \
     else if (mode == kDecS4G) ZT_GU_MODE(CPW_, TPW_, kDecS4G);                             \
     else ZT_GU_MODE(CPW_, TPW_, kDecU4G);                                                  \
