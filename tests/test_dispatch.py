@@ -42,9 +42,9 @@ def test_general_modes_17_to_64_rows():
              for kind in (dict(s_dtype="float32"), dict(zp="bfloat16"), dict(zp="int32"))
              for M, K, N, prefill in [
                  (17, 4096, 4096, False), (32, 2048, 2048, False), (24, 4096, 512, False),
-                 (32, 256, 256, False), (24, 2048, 1001, False), (33, 4096, 4096, False),
+                 (32, 512, 512, False), (24, 2048, 1001, False), (33, 4096, 4096, False),
                  (64, 4096, 4096, True), (48, 4096, 14336, True), (24, 3584, 18944, True),
-                 (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 256, 256, True)]]
+                 (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 512, 512, True)]]
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert lines and lines[0].startswith("woq prefill") == prefill, (call, lines)
 
@@ -67,3 +67,17 @@ def test_gate_up_large_tiles_or_two_steps():
               (dict(M=64, K=3584, N=37888, gate_up=True, zp="bfloat16"), True)]
     for (call, merged), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert any(l.endswith(", gate_up") for l in lines) == merged, (call, lines)
+
+
+# short K at up to 64 rows: the synchronous kernel (it prints no launch line),
+# the large tiles past its limits
+def test_short_k_kernel():
+    cases = [(dict(M=M, K=K, N=256, **kind), prefill)
+             for kind, limit in ((dict(gs=32), 320), (dict(gs=64), 320),
+                                 (dict(gs=32, zp="int8"), 256), (dict(gs=64, s_dtype="float32"), 256))
+             for M, K, prefill in [(1, 64, False), (16, 192, False), (64, 192, False),
+                                   (16, 256, False), (64, 320, limit < 320), (16, 320, limit < 320),
+                                   (16, 384, True), (65, 64, True)]]
+    for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert any(l.startswith("woq prefill") for l in lines) == prefill, (call, lines)
+        assert prefill or not lines, (call, lines)

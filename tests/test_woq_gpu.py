@@ -859,3 +859,15 @@ def test_prefill_strided_operands(variant, op_dtype, M, N, ld, knobs):
     y = C.woq_linear(xs[:, :K], wd, sd, None, bd, post_ops=("mul", "add"),
                      post_bufs=[d[:, :N] for d in big])
     check_close(y, y_ref)
+
+
+# K that gives a wave of the stream kernel two chunks or fewer, and the
+# synchronous kernel up to 64 rows of K = 256 (zero points) or 320
+@pytest.mark.parametrize("M,K,N", [(1, 1024, 40), (8, 64, 36), (16, 192, 260), (33, 192, 68),
+                                   (9, 256, 132), (64, 320, 36), (2, 2048, 100)])
+@pytest.mark.parametrize("gs,zp", [(64, torch.uint8), (64, None), (32, torch.int8), (32, None)])
+def test_group_modes_short_k(M, K, N, gs, zp):
+    x, wp, s, z, b = group_case(M, K, N, gs, zp, M + K + N + gs)
+    y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b, post_ops=("relu",))
+    xd, wd, sd, zd, bd = gpu(x, wp, s, z, b)
+    check_close(C.woq_linear(xd, wd, sd, zd, bd, post_ops=("relu",)), y_ref)

@@ -352,7 +352,10 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   {
     const char *f = zt::knob(zt::kKnobWoqForceKernel);
     hipError_t err = hipSuccess;
-    if ((!f || !std::strcmp(f, "decode")) && zt::woq_try_group_stream(a, s, &err))
+    // (many columns of a short K re-read x for every row tile: 28672 x 256 at
+    // M = 32 / 64 8.7 / 13.1 us on the stream kernel, 7.6 / 8.1 on the synchronous one)
+    const bool rereads = !f && M > kWoqRowBlock && M * N > (1 << 19) && zt::woq_short_k(a);
+    if ((!f || !std::strcmp(f, "decode")) && !rereads && zt::woq_try_group_stream(a, s, &err))
       return hip_status(err, op);
   }
   // 17..64 rows with fp32 scales or zero points the wide kernel does not
@@ -361,10 +364,13 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   // dequantisation per row block
   if (M > kWoqRowBlock && M <= kWoqRowBlockMax && (zp || scales_dtype == ZT_DT_F32) &&
       !zt::knob(zt::kKnobWoqForceKernel) && !zt::knob(zt::kKnobWoqStream) &&
-      zt::woq_prefill_ok(a) &&
-      zt::woq_prefill_workspace(M, N, K) <= (workspace ? workspace_bytes : 0) &&
-      (!woq_use_row_blocks(a) || zt::woq_prefill_beats_row_blocks(a)))
-    return hip_status(zt::launch_woq_prefill(a, false, workspace, workspace_bytes, s), op);
+      zt::woq_prefill_ok(a)) {
+    if (zt::woq_short_k(a))
+      return hip_status(zt::launch_woq_gemm(a, s, workspace, workspace_bytes), op);
+    if (zt::woq_prefill_workspace(M, N, K) <= (workspace ? workspace_bytes : 0) &&
+        (!woq_use_row_blocks(a) || zt::woq_prefill_beats_row_blocks(a)))
+      return hip_status(zt::launch_woq_prefill(a, false, workspace, workspace_bytes, s), op);
+  }
   if (woq_use_row_blocks(a)) {
     // one stream-kernel launch over all rows when x (in K phases) fits, else
     // blocks of 16 rows

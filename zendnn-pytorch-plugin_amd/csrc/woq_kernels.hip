@@ -2834,6 +2834,16 @@ size_t woq_gemm_workspace(int64_t M, int64_t N, int64_t K) {
                   woq_prefill_workspace(M, N, K));
 }
 
+// Up to 64 rows of a few steps of K the synchronous kernel's short prologue
+// wins over the large tiles' whole row tile (graph replays, 16 / 64 rows of 1024
+// columns: K = 64 3.8 / 4.2 us against 5.2 / 6.4, 256 6.0 / 6.7 against 6.8, 320 6.9 /
+// 7.6 against 7.3 / 8.4, 384 7.7 against 7.8; zero points and fp32 scales, which
+// it dequantises by two operations, K = 192 6.2 / 6.8 against 6.7 / 7.9, 256 7.4 against
+// 7.3, 320 8.6 against 7.9)
+bool woq_short_k(const WoqArgs &a) {
+  return a.M <= 64 && a.K <= (a.zp || a.s_dt == ZT_DT_F32 ? 256 : 320);
+}
+
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {
   return launch_woq_gemm(a, s, nullptr, 0);
 }
@@ -2842,7 +2852,7 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace, siz
   if (a.M == 0 || a.N == 0) return hipSuccess;
   // o: the synchronous kernel, v / w / x: load waves, else the large tiles
   const char *e = knob(kKnobWoqGemm);
-  if (woq_prefill_ok(a) && !(e && e[0] == 'o')) {
+  if (woq_prefill_ok(a) && (e ? e[0] != 'o' : !woq_short_k(a))) {
     // The load-wave kernel where it is ahead of the large-tile kernel: one
     // round of its 256 x 128 tiles at least three quarters full over at most
     // two row tiles, where the weights come from HBM and its third stage hides

@@ -56,6 +56,8 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s);
 // with less it runs unsplit.
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace,
                            size_t workspace_bytes);
+// Whether launch_woq_gemm takes its synchronous kernel for a short K.
+bool woq_short_k(const WoqArgs &a);
 // Large-tile prefill GEMM (woq_prefill.hip): whether it takes these
 // operands, the tile and K split it takes for a shape (tile 0: 128 x 128, 1:
 // 128 x 256, 2: 256 x 256; us: the estimate they were chosen by), the bytes of
