@@ -81,3 +81,17 @@ def test_short_k_kernel():
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert any(l.startswith("woq prefill") for l in lines) == prefill, (call, lines)
         assert prefill or not lines, (call, lines)
+
+
+# merged gate_up without its workspace: taken by the decode kernels' one launch
+# for signed weights in groups of 128 and up, refused for all others
+def test_gate_up_short_workspace():
+    cases = [(dict(M=M, K=4096, N=28672, gate_up=True, workspace=ws, **kind), ok)
+             for kind, ok in ((dict(), True), (dict(zp="int8"), False), (dict(gs=64), False),
+                              (dict(gs=32, zp="uint8"), False))
+             for M in (1, 12, 24) for ws in (0, 4 * M * 28672 - 256)]
+    cases += [(dict(M=M, K=4096, N=28672, gate_up=True, workspace=4 * M * 28672, zp="int8"), True)
+              for M in (1, 12, 24)]
+    cases += [(dict(M=200, K=4096, N=28672, gate_up=True, workspace=0), False)]
+    for (call, ok), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert ("workspace of" not in status) == ok, (call, status, lines)

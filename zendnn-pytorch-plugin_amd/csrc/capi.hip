@@ -430,12 +430,16 @@ int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   a.y = y, a.y_dt = y_dtype, a.ldy = ldy;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   hipError_t err = hipSuccess;
-  if (zt::woq_try_stream_gate_up(a, s, &err)) return hip_status(err, op);
-  if (zt::woq_try_wide_gate_up(a, s, &err)) return hip_status(err, op);
-  // the full [M, N] in fp32, asked of every call past the decode kernels:
-  // whether a shape needs it is not the caller's to know
+  // the full [M, N] in fp32, asked of every call but the signed ones in groups
+  // of 128 and up that the decode kernels take in one launch: whether a shape
+  // needs it is not the caller's to know
   const size_t h = ((size_t)M * (size_t)N * sizeof(float) + 255) / 256 * 256;
-  if (!workspace || workspace_bytes < h)
+  const bool room = workspace && workspace_bytes >= h;
+  if (room || (!zp && (G == 1 || (K / G) % 128 == 0))) {
+    if (zt::woq_try_stream_gate_up(a, s, &err)) return hip_status(err, op);
+    if (zt::woq_try_wide_gate_up(a, s, &err)) return hip_status(err, op);
+  }
+  if (!room)
     return fail(ZT_EINVAL, "%s: workspace of %zu bytes needed, %zu given", op,
                 zt_woq_linear_gate_up_workspace_size(M, K, N, G),
                 workspace ? workspace_bytes : (size_t)0);
