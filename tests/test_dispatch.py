@@ -95,3 +95,15 @@ def test_gate_up_short_workspace():
     cases += [(dict(M=200, K=4096, N=28672, gate_up=True, workspace=0), False)]
     for (call, ok), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert ("workspace of" not in status) == ok, (call, status, lines)
+
+
+# bf16 scales that start in the middle of a dword keep zero points and small
+# groups off the kernels that move them by 4-byte DMA
+def test_misaligned_scales():
+    calls = [dict(M=M, K=4096, N=28672, gate_up=gu, scales=(1 << 20) + at, **kind)
+             for kind in (dict(zp="int8"), dict(gs=64), dict(gs=32, zp="uint8"))
+             for M in (4, 24, 64) for gu in (False, True) for at in (0, 2)]
+    for call, (status, lines) in zip(calls, plans(calls)):
+        staged = any(l.startswith(("woq wide", "woq gate_up stream")) for l in lines) or \
+            any(l.startswith("woq stream") for l in lines) and "zp" not in call
+        assert lines and (call["scales"] % 4 == 0 or not staged), (call, lines)

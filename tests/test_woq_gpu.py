@@ -871,3 +871,20 @@ def test_group_modes_short_k(M, K, N, gs, zp):
     y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b, post_ops=("relu",))
     xd, wd, sd, zd, bd = gpu(x, wp, s, z, b)
     check_close(C.woq_linear(xd, wd, sd, zd, bd, post_ops=("relu",)), y_ref)
+
+
+# scales and zero points that start at odd elements of their buffers
+@pytest.mark.parametrize("M", [4, 24, 64, 130])
+@pytest.mark.parametrize("gs,zp", [(128, torch.int8), (64, None), (32, torch.uint8)])
+def test_misaligned_scales(M, gs, zp):
+    K, N = 2048, 4164
+    x, wp, s, z, b = group_case(M, K, N, gs, zp, M + gs)
+    y_ref = O.woq_linear(x, wp, s, zero_points=z, bias=b)
+    def odd(t):
+        if t is None:
+            return None
+        buf = torch.zeros(t.numel() + 1, dtype=t.dtype, device=DEV)
+        buf[1:] = t.flatten().to(DEV)
+        return buf[1:].view(t.shape)
+    xd, wd, bd = gpu(x, wp, b)
+    check_close(C.woq_linear(xd, wd, odd(s), odd(z), bd), y_ref)

@@ -2588,6 +2588,10 @@ bool woq_wide_ok(const WoqArgs &a, WidePlan *p) {
   if (a.zp && ((a.zp_dt != ZT_DT_S8 && a.zp_dt != ZT_DT_U8) ||
                (reinterpret_cast<uintptr_t>(a.zp) & 3u)))
     return false;
+  // their scales, and those of groups of 32 and 64: whole dwords too (as in
+  // group_mode; other kernels load them one by one)
+  if ((a.zp || (a.G > 1 && a.K / a.G < 128)) && (reinterpret_cast<uintptr_t>(a.scales) & 3u))
+    return false;
   return a.x_dt == ZT_DT_BF16 && a.s_dt == ZT_DT_BF16 && a.ldx % 8 == 0 && aligned16(a.x) && aligned16(a.w) &&
          (a.M - 1) * a.ldx * 2 + a.K * 2 < (int64_t)kOobOffset &&
          a.N * (a.K / 2) < (int64_t)kOobOffset && a.G * a.N * 2 < (int64_t)kOobOffset;
