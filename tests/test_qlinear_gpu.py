@@ -199,3 +199,16 @@ def test_qlinear_requantised_large_m(kind, N, post, knobs):
     y = op(*dev(x, w, xs, xz, ws, None, b, ys, yz), output_dtype=torch.uint8)
     check(y, O.qlinear(x, w, xs, xz, ws, b, post_ops=post, out_dtype=torch.uint8, y_scale=ys,
                        y_zp=yz))
+
+
+# both static quantise kernels, at the edges of their rule (one element per
+# thread up to 128 rows of 256 bf16 or fp32 values, else sixteen): rows and K
+# on either side, K in and not in whole sixteens, row-major and fragment order
+@pytest.mark.parametrize("in_dtype", [torch.float32, torch.bfloat16, torch.uint8, torch.int8])
+@pytest.mark.parametrize("M,K", [(1, 16), (1, 256), (100, 256), (128, 256), (129, 256), (128, 272),
+                                 (33, 192), (5, 250), (200, 264), (130, 4096)])
+def test_qlinear_quantise_kernels(M, K, in_dtype):
+    x, w, xs, xz, ws, b = make(M + K, shape=(M, K), N=36, in_dtype=in_dtype)
+    y = ops.zentorch_qlinear(*dev(x, w, xs, xz, ws, None, b, None, None),
+                             output_dtype=torch.float32)
+    check(y, O.qlinear(x, w, xs, xz, ws, b, out_dtype=torch.float32))
