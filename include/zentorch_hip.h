@@ -97,14 +97,16 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
                   int32_t y_dtype, int64_t ldy, void *workspace,
                   size_t workspace_bytes, zt_stream_t stream);
 
-/* Bytes of device workspace zt_woq_linear needs for these sizes.  Calls that
- * split K over several workgroups keep fp32 partials [splits][M][N] there
+/* Bytes of device workspace zt_woq_linear takes for these sizes: an upper
+ * bound over the scale and zero-point types, which it does not ask for.  Calls
+ * that split K over several workgroups keep fp32 partials [splits][M][N] there
  * (no initial contents needed): 17..64 rows on large matrices (and from 4
  * rows where the decode kernels have no good layout for x, e.g. K = 11008
  * at 15-16 rows; a smaller workspace is refused for these), and prefill
  * calls, also those of 17..64 rows with zero points or fp32 scales, whose
  * estimated time a K split shortens (a smaller workspace runs those
- * unsplit, or on the decode kernels); other sizes need none (0).  A split
+ * unsplit, or on the decode kernels).  Signed bf16-scale calls of 17..64 rows
+ * on smaller matrices never touch it; other sizes need none (0).  A split
  * keeps rows of N rounded up to a multiple of 4.  Calls that
  * overlap in time must not share a workspace. */
 size_t zt_woq_linear_workspace_size(int64_t M, int64_t K, int64_t N,
@@ -122,11 +124,14 @@ size_t zt_woq_linear_workspace_size(int64_t M, int64_t K, int64_t N,
  * u = zt_woq_linear(x, W[I:2I]) then zt_woq_linear(x, W[0:I]) with the
  * post-ops {SILU, MUL u}.  Arguments as zt_woq_linear without post-ops;
  * N even, y [M, ldy] with N/2 columns.  Pass a workspace of
- * zt_woq_linear_gate_up_workspace_size(M, K, N, G) bytes on every call:
- * calls the fused kernels take (bf16 x and scales, no zero points, up to 64
- * rows, I % 16 == 0, x within the kernel's LDS, no K split) run as one
- * launch and leave it untouched; the others run the full linear into fp32
- * there, then the epilogue.
+ * zt_woq_linear_gate_up_workspace_size(M, K, N, G) bytes on every call.
+ * Signed weights in groups of 128 and up that the fused decode kernels take
+ * (bf16 x and scales, up to 64 rows, I % 16 == 0, x within the kernel's LDS, no
+ * K split) run as one launch without it; every other call is refused with
+ * less than the fp32 [M, N] result.  Those that no kernel takes in one launch
+ * (the decode kernels also take 8-bit zero points and groups of 32 and 64, the
+ * prefill kernel what it would not split) run the full linear into it, then
+ * the epilogue.
  */
 int zt_woq_linear_gate_up(const void *x, int32_t x_dtype, int64_t M, int64_t K,
                           int64_t ldx, const int32_t *w_packed, int64_t N,

@@ -599,10 +599,11 @@ def test_persist_kernel_gate_up_strided_x():
     assert torch.equal(y, y0)
 
 
-# every prefill GEMM variant by name (ZT_WOQ_GEMM): "w" / "v" / "x" the
-# load-wave kernel, "o" the synchronous kernel, any other the large-tile kernel
-# unsplit; ragged M and N, two scale dtypes
-@pytest.mark.parametrize("variant", ["1", "w", "v", "x", "d", "2", "o"])
+# every prefill GEMM by name (ZT_WOQ_GEMM): "w" the load-wave kernel (the large
+# tiles where it does not take fp32 scales), "o" the synchronous kernel, "p<tile>"
+# the large tiles as the plan splits them and unsplit; ragged M and N, two scale
+# dtypes
+@pytest.mark.parametrize("variant", ["w", "o", "p0", "p01", "p11", "p21"])
 @pytest.mark.parametrize("M,K,N,G,s_dtype", [(300, 1024, 264, 8, torch.bfloat16),
                                              (520, 2048, 520, 16, torch.bfloat16),
                                              (97, 512, 136, 4, torch.float32)])
@@ -615,9 +616,9 @@ def test_prefill_gemm_variants(variant, M, K, N, G, s_dtype):
     check_close(y, y_ref)
 
 
-# post-ops in the prefill variants' epilogues (the large-tile and the load-wave
-# kernel), with bias, elementwise and binary post-ops
-@pytest.mark.parametrize("variant", ["1", "w", "x", "2"])
+# post-ops in the epilogues of the load-wave kernel, the large tiles and their
+# splits' reduction, with bias, elementwise and binary post-ops
+@pytest.mark.parametrize("variant", ["w", "p01", "p11", "p21", "p04"])
 @pytest.mark.parametrize("post,nbuf", [(("gelu_erf",), 0), (("mul", "add"), 2),
                                        (("silu", "mul"), 1)])
 def test_prefill_variants_post_ops(variant, post, nbuf):
@@ -632,20 +633,13 @@ def test_prefill_variants_post_ops(variant, post, nbuf):
     check_close(y, y_ref)
 
 
-# the default prefill dispatch at half a round of 256 x 128 tiles
-def test_prefill_one_round_default_kernel():
-    M, K, N, G = 2048, 256, 2048, 2
+# the default prefill dispatch: many row tiles over few columns, more than one
+# round of the largest tiles with ragged M, and the one nearly full round of 256 x
+# 128 tiles over two row tiles (198 of them) that the load-wave kernel takes
+@pytest.mark.parametrize("M,K,N,G", [(2048, 256, 2048, 2), (2100, 256, 4608, 2),
+                                     (300, 256, 12552, 2)])
+def test_prefill_default_kernel(M, K, N, G):
     x, q, wp, s, z, b = make_case(M, K, N, G, seed=11, bias=True)
-    y_ref = O.woq_linear(x, wp, s, bias=b)
-    xd, wd, sd, bd = gpu(x, wp, s, b)
-    y = C.woq_linear(xd, wd, sd, None, bd)
-    check_close(y, y_ref)
-
-
-# ragged M over more than one round of 256 x 128 tiles (9 x 36 = 324)
-def test_prefill_one_round_192_default_kernel():
-    M, K, N, G = 2100, 256, 4608, 2
-    x, q, wp, s, z, b = make_case(M, K, N, G, seed=12, bias=True)
     y_ref = O.woq_linear(x, wp, s, bias=b)
     xd, wd, sd, bd = gpu(x, wp, s, b)
     y = C.woq_linear(xd, wd, sd, None, bd)
@@ -836,7 +830,7 @@ def test_zero_points_scale_range(M, N, force, big, zp, z0, gs, knobs):
 # x and binary post-op operands with rows longer than K and N on the large tiles
 # (every tile, and the load-wave kernel): fp32 and bf16 operands whose rows are
 # and are not whole 16- or 8-byte pieces, ragged M and N
-@pytest.mark.parametrize("variant", ["p01", "p11", "p21", "p03", "v"])
+@pytest.mark.parametrize("variant", ["p01", "p11", "p21", "p03", "w"])
 @pytest.mark.parametrize("op_dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,ld", [(130, 264, 264), (300, 264, 272), (130, 264, 267)])
 def test_prefill_strided_operands(variant, op_dtype, M, N, ld, knobs):

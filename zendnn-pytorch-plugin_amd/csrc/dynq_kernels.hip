@@ -100,10 +100,11 @@ __device__ __forceinline__ void block_minmax(float &lo, float &hi, float *red, i
 }
 
 // The quantise kernels also clear the tile counters of the split-K GEMM that
-// follows them on the stream (workgroup 0, 256 threads).
+// follows them on the stream (workgroup 0, NT threads).
+template <int NT = 256>
 __device__ __forceinline__ void zero_counters(int32_t *zero, int nzero, int tid) {
   if (blockIdx.x == 0)
-    for (int i = tid; i < nzero; i += 256) zero[i] = 0;
+    for (int i = tid; i < nzero; i += NT) zero[i] = 0;
 }
 
 template <bool ASYM>
@@ -172,7 +173,7 @@ __global__ __launch_bounds__(NT) void dyn_quantize_vec_kernel(const typename V::
   __shared__ float red[NT / 32];
   const int tid = threadIdx.x;
   const int64_t m = blockIdx.x;
-  zero_counters(zero, nzero, tid);
+  zero_counters<NT>(zero, nzero, tid);
   const typename V::elem *row = x + m * K;
   const int nv = (int)(K / 8);
   V v[VPT];
@@ -507,8 +508,10 @@ __device__ __forceinline__ void dyn_epilogue4(const DynArgs &a, int m, int n, i3
 // 256 threads.  BN/4 divides 256, so each thread keeps the same four columns
 // for all its rows: their weight scales and bias are loaded once, and the
 // row scales come from LDS (sx_l).  Same arithmetic as dyn_epilogue:
-// ((float)acc * sx[m]) * sw[n] + bias[n].  Post-ops, int32 output and a row
-// length that is not a multiple of 4 take the general path.
+// ((float)acc * sx[m]) * sw[n] + bias[n].  Post-ops, requantised outputs and a
+// row length that is not a multiple of 4 take whole passes over the tile where
+// NT / G4 rows divide BM (all but the 256 x 192 tile); int32 outputs and that tile
+// the general path, quad by quad.
 template <int BM, int BN, int NT = 256>
 __device__ __forceinline__ void s8_tile_epilogue(const DynArgs &a, const int32_t *tile,
                                                  const float *sx_l, int m0, int n0, int tid) {
@@ -2380,10 +2383,10 @@ hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s) {
                    ? launch_s8_ws<128, 128, 2, 2, 4, 3>(a, s, a.gemm_splits)
                    : launch_s8_ws<128, 128, 2, 2, 4, 3>(a, s);
       }
+      if (!tile && !kind && s8_prefill_better(a.M, a.N, a.K)) return launch_s8_prefill(a, s);
       // 256 x 192 tiles (six compute waves of 128 x 64, two load waves, two
       // stages) where they make one round and 256 x 128 tiles do not: QKV at
       // M = 2048, 256 against 384 tiles, 69 -> 58.5 us
-      if (!tile && !kind && s8_prefill_better(a.M, a.N, a.K)) return launch_s8_prefill(a, s);
       const int64_t t192 = ((a.M + 255) / 256) * ((a.N + 191) / 192);
       const bool w192 = tile ? tile[0] == '9' : t256 > 256 && t192 <= 256;
       if (w192) return launch_s8_ws<256, 192, 2, 3, 2, 2>(a, s);

@@ -49,7 +49,6 @@ void s8_prefill_kernel(DynArgs a, int tiles_m, int tiles_n, int group_m) {
   const int M = (int)a.M, N = (int)a.N, K = (int)a.K;
   const int m0 = tm * BM, n0 = tn * BN;
   const int nk = (K + kPqBK - 1) / kPqBK;
-  const int tail = K % kPqBK ? nk - 1 : -1;            // the step that ends inside a row
 
   // rows of the [x | W] slab, 8 per load, 16-byte chunk c of row r at
   // c ^ ((r >> 1) & 7); a load lies wholly in x or in W
@@ -240,7 +239,9 @@ bool s8_prefill_better(int64_t M, int64_t N, int64_t K) {
   // the load-wave kernel's 256 x 192 tiles where they make one round and its
   // 256 x 128 do not: 1-3 % ahead up to K = 4096 (quantisation included, M =
   // 2048: 6144 x 2048 42.4 against 43.3 us, 5120 x 4096 59.7 against 61.1),
-  // behind past it (5120 x 5120 81.0 against 75.3, 6144 x 8192 120.7 against 118)
+  // behind past it (5120 x 5120 81.0 against 75.3, 6144 x 8192 120.7 against 118).
+  // All without post-ops and with bf16 outputs: post-ops and requantised outputs
+  // go quad by quad in that tile's epilogue (s8_tile_epilogue), pass by pass here.
   if (tm * ((N + 127) / 128) > 256 && tm * ((N + 191) / 192) <= 256 && K <= 4096) return false;
   return rounds_us(tm * ((N + 255) / 256), nk, 11.0, 1.10, 1.72) <
          rounds_us(tm * ((N + 127) / 128), nk, 8.0, 0.70, 0.98);

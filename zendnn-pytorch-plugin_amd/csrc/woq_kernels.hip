@@ -31,13 +31,14 @@
 //    not take (long K split over workgroups, general dequant modes).
 //  * woq_prefill_kernel (woq_prefill.hip)  more rows than the decode kernels
 //    take, groups of 32 and up, any zero-point and scale type; also 17..64
-//    rows with zero points or fp32 scales, and any row count in groups of 32
-//    and 64.
+//    rows with zero points or fp32 scales where it beats blocks of 16 rows, and
+//    any row count in groups of 32 and 64 that the decode kernels leave.
 //  * woq_gemm_ws_kernel  one nearly full round of 256 x 128 tiles at up to
 //    512 rows (signed int4, bf16 scales): loads in waves of their own, three
 //    stages.
-//  * woq_gemm_kernel  synchronous tiles for what the 32-bit offsets, x types,
-//    alignment and group sizes of woq_prefill_kernel exclude.
+//  * woq_gemm_kernel  synchronous tiles: up to 64 rows of a short K, and what
+//    the 32-bit offsets, x types, alignment and group sizes of
+//    woq_prefill_kernel exclude.
 //  * woq_generic_kernel  what none of the above takes (K not a multiple of
 //    64, odd group sizes): one wave per output element.
 //
@@ -2820,9 +2821,10 @@ hipError_t launch_woq_decode(const WoqArgs &a, const DecodePlan &p, void *worksp
   return hipErrorInvalidValue;
 }
 
-// K splits of the prefill GEMM when its 128 x 128 tiles (the tile it takes
-// at half a round of 256 x 128 tiles or less) make at most one round: up to
-// 8, about two workgroups per CU, at least 16 steps of 64 each (1 = no split)
+// The most K splits of a prefill call whose 128 x 128 tiles make at most one
+// round (and 256 x 128 ones half a round): up to 8, about two workgroups per CU,
+// at least 16 steps of 64 each (1 = not such a call).  woq_prefill_plan takes no
+// more of them and woq_gemm_workspace reports no fewer bytes.
 int woq_gemm_splits(int64_t M, int64_t N, int64_t K) {
   if (M < 1 || N < 1 || K < 1 || knob(kKnobWoqGemm)) return 1;
   const int64_t t256 = ((M + 255) / 256) * ((N + 127) / 128);
@@ -2854,7 +2856,7 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {
 
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace, size_t workspace_bytes) {
   if (a.M == 0 || a.N == 0) return hipSuccess;
-  // o: the synchronous kernel, v / w / x: load waves, else the large tiles
+  // o: the synchronous kernel, w: load waves, else the large tiles
   const char *e = knob(kKnobWoqGemm);
   if (woq_prefill_ok(a) && (e ? e[0] != 'o' : !woq_short_k(a))) {
     // The load-wave kernel where it is ahead of the large-tile kernel: one
@@ -2866,8 +2868,7 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace, siz
     const int64_t cpg = a.K / a.G / 128, tiles = ((a.M + 255) / 256) * ((a.N + 127) / 128);
     const bool ok = !a.zp && a.s_dt == ZT_DT_BF16 && a.N % 8 == 0 && a.K % 128 == 0 &&
                     (a.G == 1 || (a.K / a.G) % 128 == 0);
-    const bool load_wave = e ? e[0] == 'v' || e[0] == 'w' || e[0] == 'x'
-                             : a.M <= 512 && tiles > 192 && tiles <= 256;
+    const bool load_wave = e ? e[0] == 'w' : a.M <= 512 && tiles > 192 && tiles <= 256;
     if (!ok || !load_wave) return launch_woq_prefill(a, false, workspace, workspace_bytes, s);
     int shift = 0;
     while (cpg > 1 && (1 << shift) < cpg) ++shift;

@@ -24,12 +24,14 @@ __device__ __forceinline__ i32x4_t dma_rsrc(const void *p, uint32_t bytes) {
 }
 
 // One 16-byte-per-lane load of buffer bytes voff + soff straight into LDS at
-// lds + 16 * lane; a lane whose voff is kOobOffset gets zeros.  Written as assembly because the compiler,
-// seeing the builtin, waits for every such load in flight before each later
+// lds + 16 * lane; a lane whose voff is kOobOffset gets zeros.  Written as
+// assembly because the compiler, seeing the builtin, waits for every such load in flight before each later
 // LDS read it cannot prove disjoint (vmcnt(0) in the middle of the step that
 // the loads were issued ahead of); it has no register result, and the
 // callers wait for it themselves (wait_step) before the barrier that
-// publishes the stage.  Writing M0 needs one wait state before the load.
+// publishes the stage.  Writing M0 needs one wait state before the load; the
+// kernels that call this hold nothing else in M0 (it cannot be named as a
+// clobber: the compiler reserves it), so they use no builtin that does.
 __device__ __forceinline__ void dma16(i32x4_t rsrc, uint32_t lds, uint32_t voff, uint32_t soff) {
   asm volatile("s_mov_b32 m0, %0\n\t"
                "s_nop 0\n\t"
