@@ -76,8 +76,8 @@ def test_short_k_kernel():
              for kind, limit in ((dict(gs=32), 320), (dict(gs=64), 320),
                                  (dict(gs=32, zp="int8"), 256), (dict(gs=64, s_dtype="float32"), 256))
              for M, K, prefill in [(1, 64, False), (16, 192, False), (64, 192, False),
-                                   (16, 256, False), (64, 320, limit < 320), (16, 320, limit < 320),
-                                   (16, 384, True), (65, 64, True)]]
+                                   (64, 320, limit < 320), (16, 320, limit < 320),
+                                   (16, 448, True), (65, 64, True)]]
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert any(l.startswith("woq prefill") for l in lines) == prefill, (call, lines)
         assert prefill or not lines, (call, lines)
@@ -107,3 +107,14 @@ def test_misaligned_scales():
         staged = any(l.startswith(("woq wide", "woq gate_up stream")) for l in lines) or \
             any(l.startswith("woq stream") for l in lines) and "zp" not in call
         assert lines and (call["scales"] % 4 == 0 or not staged), (call, lines)
+
+
+# 8-bit zero points and groups of 32 and 64 at up to 16 rows take the stream
+# kernel at every whole number of 128-column chunks, short K included
+def test_group_modes_take_the_stream_kernel():
+    calls = [dict(M=M, K=128 * C, N=N, gate_up=gu, **kind)
+             for M in (1, 5, 16) for C in (1, 2, 5, 8, 9, 16, 17, 32) for N, gu in ((96, False),
+                                                                                  (9216, True))
+             for kind in (dict(gs=64), dict(gs=32), dict(gs=128, zp="int8"), dict(gs=0, zp="uint8"))]
+    for call, (status, lines) in zip(calls, plans(calls)):
+        assert len(lines) == 1 and " stream " in lines[0], (call, lines)

@@ -750,7 +750,7 @@ def group_case(M, K, N, gs, zp, seed):
 
 
 GROUP_CASES = [
-    (1, 2176, 40, "stream"), (4, 3584, 132, "stream"), (16, 4096, 260, "stream"),
+    (1, 1024, 40, "stream"), (2, 256, 36, "stream"), (4, 3584, 132, "stream"), (16, 4096, 260, "stream"),
     (9, 14336, 68, "stream"), (3, 2176, 36, "stream"), (30, 4096, 260, "stream"),
     (64, 2048, 132, "stream"), (17, 11008, 1540, "wide"), (33, 3584, 4164, "wide"),
     (64, 1280, 4164, "wide"), (12, 13824, 5124, "wide"), (17, 11008, 136, "prefill")]
@@ -855,8 +855,8 @@ def test_prefill_strided_operands(variant, op_dtype, M, N, ld, knobs):
     check_close(y, y_ref)
 
 
-# K that gives a wave of the stream kernel two chunks or fewer, and the
-# synchronous kernel up to 64 rows of K = 256 (zero points) or 320
+# K of two chunks per wave of the stream kernel and fewer, and the synchronous
+# kernel up to 64 rows of K = 256 (zero points) or 320
 @pytest.mark.parametrize("M,K,N", [(1, 1024, 40), (8, 64, 36), (16, 192, 260), (33, 192, 68),
                                    (9, 256, 132), (64, 320, 36), (2, 2048, 100)])
 @pytest.mark.parametrize("gs,zp", [(64, torch.uint8), (64, None), (32, torch.int8), (32, None)])

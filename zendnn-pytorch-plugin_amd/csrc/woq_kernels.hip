@@ -2066,9 +2066,18 @@ static bool try_launch_stream(const WoqArgs &a, hipStream_t s, int shift, int gm
   }
   if (!fits(1)) return false;
   const int need = (C + nw - 1) / nw;
+  // (two chunks per wave are built with four tiles only; K of 2048 and less leaves
+  // the fast mode's calls to the kernels above and the decode kernel, while the
+  // group modes have no other decode kernel and take four: 4096 x 2048 in groups
+  // of 64 at M = 1 / 16 14.6 / 15.1 us on the large tiles, 4.0 / 4.8 here; with
+  // 8-bit zero points in groups of 128 5.8 / 7.5 in the general mode, 4.1 / 4.8)
+  const bool group = mode == kDecS4G || mode == kDecU4G;
   if (cpw == 0)
     for (int c : {2, 4, 8, 12, 14, 16, 28})
-      if (c >= need && ((c != 14 && c != 28) || nw == 8)) { cpw = c; break; }
+      if (c >= need && ((c != 14 && c != 28) || nw == 8) && (c > 2 || tpw == 4 || !group)) {
+        cpw = c;
+        break;
+      }
   if (cpw < need) return false;
 #define ZT_STREAM_CASE(NW_, CPW_, TPW_) \
   if (nw == NW_ && cpw == CPW_ && tpw == TPW_) { \
@@ -2736,7 +2745,7 @@ bool woq_try_stream_gate_up(const WoqArgs &a, hipStream_t s, hipError_t *err) {
   const int need = (C + 7) / 8;
   int cpw = 0;
   for (int c : {2, 4, 8, 12, 14, 16})
-    if (c >= need) { cpw = c; break; }
+    if (c >= need && (c > 2 || tpw == 4 || mode == kDecFast)) { cpw = c; break; }
   if (cpw < need) return false;
   const int x_dma = stream_x_dma(a, 1) ? 1 : 0;
   const dim3 grid((unsigned)((I / 16 + tpw / 2 - 1) / (tpw / 2))), block(512);
