@@ -882,3 +882,20 @@ def test_misaligned_scales(M, gs, zp):
         return buf[1:].view(t.shape)
     xd, wd, bd = gpu(x, wp, b)
     check_close(C.woq_linear(xd, wd, odd(s), odd(z), bd), y_ref)
+
+
+# every unary post-op in the large tiles' epilogue: last tiles with 32-row pieces
+# wholly and partly past M, N that is not whole quads, a binary operand behind it
+@pytest.mark.parametrize("variant", ["p01", "p11", "p21"])
+@pytest.mark.parametrize("M,N", [(3, 261), (33, 264), (96, 259), (300, 136)])
+@pytest.mark.parametrize("op", ["relu", "silu", "sigmoid", "tanh", "gelu_erf", "gelu_tanh"])
+def test_prefill_unary_post_ops(variant, M, N, op, knobs):
+    K, G = 256, 2
+    knobs.set("ZT_WOQ_FORCE_KERNEL", "gemm")
+    knobs.set("ZT_WOQ_GEMM", variant)
+    x, q, wp, s, z, b = make_case(M, K, N, G, seed=M + N, bias=True)
+    m = torch.randn(M, N, generator=torch.Generator().manual_seed(N)).to(x.dtype)
+    y_ref = O.woq_linear(x, wp, s, bias=b, post_ops=(op, "mul"), post_bufs=[m])
+    xd, wd, sd, bd = gpu(x, wp, s, b)
+    y = C.woq_linear(xd, wd, sd, None, bd, post_ops=(op, "mul"), post_bufs=gpu(m))
+    check_close(y, y_ref)

@@ -168,6 +168,8 @@ void s8_prefill_kernel(DynArgs a, int tiles_m, int tiles_n, int group_m) {
   }
 #pragma unroll 1
   for (int i = 0; i < TM; ++i) {
+    const int mb = m0 + wm * WR + i * 32;
+    if (mb >= M) break;  // rows past M: nothing to store
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii)
       if (ii == i)
@@ -179,7 +181,6 @@ void s8_prefill_kernel(DynArgs a, int tiles_m, int tiles_n, int group_m) {
                 i32x4_t{acc[ii][j][4 * r], acc[ii][j][4 * r + 1], acc[ii][j][4 * r + 2],
                         acc[ii][j][4 * r + 3]};
     __builtin_amdgcn_wave_barrier();
-    const int mb = m0 + wm * WR + i * 32;
     auto sums = [&](int t) {
       return *reinterpret_cast<const i32x4_t *>(slab + (t * 4 + r0) * SP + c4);
     };

@@ -317,6 +317,8 @@ void woq_prefill_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int gs
   const bool has_bias = a.bias != nullptr;
 #pragma unroll 1
   for (int i = 0; i < TM; ++i) {
+    const int mb = m0 + wm * (BM / WM) + i * 32;
+    if (mb >= M) break;  // rows past M: nothing to store (few rows of a short K, last tiles)
 #pragma unroll
     for (int ii = 0; ii < TM; ++ii)
       if (ii == i)
@@ -328,9 +330,8 @@ void woq_prefill_kernel(WoqArgs a, int tiles_m, int tiles_n, int group_m, int gs
                 f32x4_t{acc[ii][j][4 * r], acc[ii][j][4 * r + 1], acc[ii][j][4 * r + 2],
                         acc[ii][j][4 * r + 3]};
     __builtin_amdgcn_wave_barrier();
-    const int mb = m0 + wm * (BM / WM) + i * 32;
     if (GU || (a.post.count && !partial)) {
-#pragma unroll 1
+#pragma unroll GU ? 1 : 4
       for (int t = 0; t < 32 / RP; ++t) {
         float *at = slab + (t * RP + r0) * SP + c4;
         f32x4_t v = *reinterpret_cast<const f32x4_t *>(at);

@@ -109,8 +109,8 @@ __device__ __forceinline__ void post_ops4(float (&f)[4], const PostOps &p, int64
 // holds column quads c4 of rows r0 + t * RP (t < T), global row mb + that and
 // column n.  Op by op over the whole slab and not quad by quad: the binary
 // operands of all T rows are then in flight together (a quad at a time each
-// waited for its own load, 32 round trips per tile), and the longer unary
-// functions' code exists once.
+// waited for its own load, 32 round trips per tile), and the unary functions'
+// code exists once for all rows.
 template <int T, int RP>
 __device__ __forceinline__ void post_ops_slab(float *slab, int pitch, int c4, int r0,
                                               const PostOps &p, int mb, int n, int M, int N) {
@@ -149,25 +149,36 @@ __device__ __forceinline__ void post_ops_slab(float *slab, int pitch, int c4, in
           apply(t, f32x4_t{bf16_bits_to_f32(o[t][0] & 0xffffu), __uint_as_float(o[t][0] & 0xffff0000u),
                            bf16_bits_to_f32(o[t][1] & 0xffffu), __uint_as_float(o[t][1] & 0xffff0000u)});
       } else {
+        // rows that are not whole aligned quads: element by element, four rows'
+        // loads in flight (columns past N read column N - 1, and are not stored)
+        auto elements = [&](auto *src) {
+          constexpr int U = T % 4 == 0 ? 4 : 1;
 #pragma unroll 1
-        for (int t = 0; t < T; ++t) {
-          float *q = slab + (t * RP + r0) * pitch + c4;
-          const int64_t at = min(mb + t * RP + r0, M - 1) * p.ld[b] + n;
+          for (int t0 = 0; t0 < T; t0 += U) {
+            f32x4_t o[U];
 #pragma unroll
-          for (int r = 0; r < 4; ++r)
-            if (n + r < N) {
-              const float w = load_elem(p.bufs[b], p.dts[b], at + r);
-              q[r] = id == ZT_PO_ADD ? q[r] + w : q[r] * w;
-            }
-        }
+            for (int t = 0; t < U; ++t)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) {
+                const auto v =
+                    src[min(mb + (t0 + t) * RP + r0, M - 1) * p.ld[b] + min(n + r, N - 1)];
+                if constexpr (sizeof(v) == 4) o[t][r] = v;
+                else o[t][r] = bf16_bits_to_f32(v);
+              }
+#pragma unroll
+            for (int t = 0; t < U; ++t) apply(t0 + t, o[t]);
+          }
+        };
+        if (f32) elements(static_cast<const float *>(p.bufs[b]));
+        else elements(static_cast<const uint16_t *>(p.bufs[b]));
       }
       ++b;
     } else {
-      // relu and silu four rows at a time: the rows' latencies overlap (one by
-      // one silu added 9 us to 14336 x 4096 at M = 200, 46 us without it); the
-      // longer functions' code stays small
-      auto rows = [&](auto count, int op) {
-        constexpr int U = T % count.value == 0 ? count.value : 1;
+      // four rows at a time, so that their latencies overlap, each function in
+      // code of its own.  Row by row a gelu, sigmoid or tanh took 12 us of a 4096 x
+      // 4096 call at M = 699 (44 us without), a silu 9 of 14336 x 4096 at M = 200.
+      auto rows = [&](auto op) {
+        constexpr int U = T % 4 == 0 ? 4 : 1;
 #pragma unroll 1
         for (int t0 = 0; t0 < T; t0 += U) {
           f32x4_t v[U];
@@ -177,14 +188,20 @@ __device__ __forceinline__ void post_ops_slab(float *slab, int pitch, int c4, in
 #pragma unroll
           for (int t = 0; t < U; ++t) {
 #pragma unroll
-            for (int r = 0; r < 4; ++r) v[t][r] = unary_op(op, v[t][r]);
+            for (int r = 0; r < 4; ++r) v[t][r] = unary_op(op.value, v[t][r]);
             *reinterpret_cast<f32x4_t *>(slab + ((t0 + t) * RP + r0) * pitch + c4) = v[t];
           }
         }
       };
-      if (id == ZT_PO_RELU) rows(std::integral_constant<int, 4>{}, ZT_PO_RELU);
-      else if (id == ZT_PO_SILU) rows(std::integral_constant<int, 4>{}, ZT_PO_SILU);
-      else rows(std::integral_constant<int, 1>{}, id);
+      switch (id) {
+      case ZT_PO_RELU: rows(std::integral_constant<int, ZT_PO_RELU>{}); break;
+      case ZT_PO_GELU_TANH: rows(std::integral_constant<int, ZT_PO_GELU_TANH>{}); break;
+      case ZT_PO_GELU_ERF: rows(std::integral_constant<int, ZT_PO_GELU_ERF>{}); break;
+      case ZT_PO_SILU: rows(std::integral_constant<int, ZT_PO_SILU>{}); break;
+      case ZT_PO_SIGMOID: rows(std::integral_constant<int, ZT_PO_SIGMOID>{}); break;
+      case ZT_PO_TANH: rows(std::integral_constant<int, ZT_PO_TANH>{}); break;
+      default: break;
+      }
     }
   }
 }
