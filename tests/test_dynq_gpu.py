@@ -430,3 +430,23 @@ def test_s8_strided_operands(kind, tile, op_dtype, ld, knobs):
     y = C.dynamic_qlinear(x.to(DEV), w.to(DEV), sw.to(DEV), b.to(DEV), post_ops=("mul", "add"),
                           post_bufs=[t.to(DEV)[:, :N] for t in bufs]).cpu()
     torch.testing.assert_close(y.float(), y_ref.float(), rtol=1e-2, atol=1e-2)
+
+
+# which large int8 kernel a call takes: 256 x 256 tiles where the load-wave kernel
+# would take its 256 x 192 ones (whose epilogue goes quad by quad) for post-ops; the
+# load-wave kernel without them, and for few k steps with a nearly empty last
+# round of 256 x 256 tiles; the same bits either way
+@pytest.mark.parametrize("M,N,K,post,prefill", [
+    (2520, 4096, 1024, (), False), (2520, 4096, 1024, ("relu",), True),
+    (2520, 4096, 1024, ("add",), True), (1346, 11264, 368, (), False),
+    (2048, 14336, 1024, (), True)])
+def test_s8_kernel_choice(M, N, K, post, prefill, knobs, capfd):
+    x, w, sw, b = make(M, K, N, seed=M + K)
+    bufs = [torch.randn(M, N, device=DEV).bfloat16() for p in post if p == "add"]
+    args = (x.to(DEV), w.to(DEV), sw.to(DEV), b.to(DEV))
+    knobs.set("ZT_WOQ_DEBUG", "1")
+    capfd.readouterr()
+    y = C.dynamic_qlinear(*args, post_ops=post, post_bufs=bufs)
+    assert ("s8 prefill" in capfd.readouterr().err) == prefill
+    knobs.set("ZT_S8_KIND", "w" if prefill else "p")
+    assert torch.equal(y, C.dynamic_qlinear(*args, post_ops=post, post_bufs=bufs))

@@ -2383,7 +2383,7 @@ hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s) {
                    ? launch_s8_ws<128, 128, 2, 2, 4, 3>(a, s, a.gemm_splits)
                    : launch_s8_ws<128, 128, 2, 2, 4, 3>(a, s);
       }
-      if (!tile && !kind && s8_prefill_better(a.M, a.N, a.K)) return launch_s8_prefill(a, s);
+      if (!tile && !kind && s8_prefill_better(a)) return launch_s8_prefill(a, s);
       // 256 x 192 tiles (six compute waves of 128 x 64, two load waves, two
       // stages) where they make one round and 256 x 128 tiles do not: QKV at
       // M = 2048, 256 against 384 tiles, 69 -> 58.5 us

@@ -43,7 +43,7 @@ struct QuadScales {
 
 // Whether the post-ops are at most one relu, which costs one instruction on
 // the way to the store and no pass of its own.
-__device__ __forceinline__ bool at_most_relu(const PostOps &p) {
+__host__ __device__ __forceinline__ bool at_most_relu(const PostOps &p) {
   return p.count == 0 || (p.count == 1 && p.ids[0] == ZT_PO_RELU);
 }
 

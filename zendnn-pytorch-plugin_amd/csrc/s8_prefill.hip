@@ -230,22 +230,29 @@ double rounds_us(int64_t wg, int64_t nk, double fixed, double few, double all) {
 
 }  // namespace
 
-// (constants from graph replays at K = 1024, 4096 and 14336 with 128 to 512
-// tiles; chosen right at all but 2 of 60 shapes of 256..4096 rows, and within 3 %
-// there)
-bool s8_prefill_better(int64_t M, int64_t N, int64_t K) {
+// (constants from graph replays of both kernels at 2743 shapes of 129 to 4096 rows,
+// K 192 to 18944: the choice is the faster kernel or within 3 % at all but 1 % of
+// those outside the 192 zone below, at most 10 % behind in it.  A tile's fixed cost
+// fitted to K >= 1024 only, 11 and 8 us, took 256 x 256 tiles for few k steps and a
+// nearly empty last round: 16460 x 784 at M = 1023 53 us against 45.  Post-ops and
+// requantised outputs lengthen the other kernel's epilogue by more.)
+bool s8_prefill_better(const DynArgs &a) {
   const char *e = knob(kKnobS8Kind);
   if (e) return e[0] == 'p';
-  const int64_t nk = (K + kPqBK - 1) / kPqBK, tm = (M + 255) / 256;
-  // the load-wave kernel's 256 x 192 tiles where they make one round and its
-  // 256 x 128 do not: 1-3 % ahead up to K = 4096 (quantisation included, M =
-  // 2048: 6144 x 2048 42.4 against 43.3 us, 5120 x 4096 59.7 against 61.1),
-  // behind past it (5120 x 5120 81.0 against 75.3, 6144 x 8192 120.7 against 118).
-  // All without post-ops and with bf16 outputs: post-ops and requantised outputs
-  // go quad by quad in that tile's epilogue (s8_tile_epilogue), pass by pass here.
-  if (tm * ((N + 127) / 128) > 256 && tm * ((N + 191) / 192) <= 256 && K <= 4096) return false;
-  return rounds_us(tm * ((N + 255) / 256), nk, 11.0, 1.10, 1.72) <
-         rounds_us(tm * ((N + 127) / 128), nk, 8.0, 0.70, 0.98);
+  const int64_t nk = (a.K + kPqBK - 1) / kPqBK, tm = (a.M + 255) / 256;
+  const bool floats = a.y_dt == ZT_DT_BF16 || a.y_dt == ZT_DT_F32;
+  // The load-wave kernel's 256 x 192 tiles where they make one round and its
+  // 256 x 128 do not: ahead up to K = 4096 (quantisation included, M = 2048: 6144 x 2048
+  // 42.4 against 43.3 us, 5120 x 4096 59.7 against 61.1), behind at most shapes past it
+  // (5120 x 5120 81.0 against 75.3, 6144 x 8192 120.7 against 118).  That tile's epilogue
+  // takes post-ops and requantised outputs quad by quad (s8_tile_epilogue): with any of
+  // them it was behind at all 267 shapes (4096 x 1024 at M = 2520 with an add 83
+  // us against 37, 14420 x 736 at M = 601 to u8 78 against 29).
+  if (tm * ((a.N + 127) / 128) > 256 && tm * ((a.N + 191) / 192) <= 256)
+    return a.K > 4096 || a.post.count || !floats;
+  const double fixed = at_most_relu(a.post) && floats ? 14.2 : 12.0;
+  return rounds_us(tm * ((a.N + 255) / 256), nk, fixed, 1.10, 1.80) <
+         rounds_us(tm * ((a.N + 127) / 128), nk, 7.1, 0.56, 1.07);
 }
 
 hipError_t launch_s8_prefill(const DynArgs &a, hipStream_t s) {

@@ -174,7 +174,7 @@ int s8_ws_splits(int64_t M, int64_t N, int64_t K);
 // Large-tile int8 GEMM (s8_prefill.hip; qx and w 16-byte aligned, K % 16 ==
 // 0, 32-bit byte offsets): whether its 256 x 256 tiles are estimated faster
 // than 256 x 128 ones on s8_gemm_ws_kernel, and the launch.
-bool s8_prefill_better(int64_t M, int64_t N, int64_t K);
+bool s8_prefill_better(const DynArgs &a);
 hipError_t launch_s8_prefill(const DynArgs &a, hipStream_t s);
 int s8_split_counters(int64_t N);
 hipError_t launch_s8_gemm(const DynArgs &a, hipStream_t s);
