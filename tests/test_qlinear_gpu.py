@@ -202,10 +202,11 @@ def test_qlinear_requantised_large_m(kind, N, post, knobs):
 
 
 # both static quantise kernels, at the edges of their rule (one element per
-# thread up to 128 rows of 256 bf16 or fp32 values, else sixteen): rows and K
+# thread up to 128 rows of 512 bf16 or fp32 values, else sixteen): rows and K
 # on either side, K in and not in whole sixteens, row-major and fragment order
 @pytest.mark.parametrize("in_dtype", [torch.float32, torch.bfloat16, torch.uint8, torch.int8])
 @pytest.mark.parametrize("M,K", [(1, 16), (1, 256), (100, 256), (128, 256), (129, 256), (128, 272),
+                                 (1, 512), (128, 512), (129, 512), (7, 528),
                                  (33, 192), (5, 250), (200, 264), (130, 4096)])
 def test_qlinear_quantise_kernels(M, K, in_dtype):
     x, w, xs, xz, ws, b = make(M + K, shape=(M, K), N=36, in_dtype=in_dtype)

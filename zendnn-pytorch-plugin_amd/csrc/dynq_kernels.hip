@@ -2250,8 +2250,9 @@ hipError_t launch_static_quantize(const void *x, int x_dt, int64_t M, int64_t K,
   if (frag && K % 64 != 0) return hipErrorInvalidValue;
   // Few short rows of bf16 or fp32 take one element per thread: sixteen in turn
   // are a longer chain than the launch has to wait for (4096 x 208 at M = 1 6.7 us
-  // in all so against 6.2, 256 x 256 at M = 32 6.5 against 6.1; equal from 200 rows)
-  const bool few = (x_dt == ZT_DT_F32 || x_dt == ZT_DT_BF16) && K <= 256 && M <= 128;
+  // in all so against 6.2, 256 x 256 at M = 32 6.5 against 6.1, 512 x 512 at M = 1 6.08
+  // against 5.76, K = 640 equal; equal from 200 rows)
+  const bool few = (x_dt == ZT_DT_F32 || x_dt == ZT_DT_BF16) && K <= 512 && M <= 128;
   if (K % 16 == 0 && !few &&
       ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(qx)) & 15u) == 0) {
     static_quantize_vec_kernel<<<dim3((unsigned)((M * (K / 16) + 255) / 256)), dim3(256), 0, s>>>(
