@@ -44,7 +44,8 @@ def test_general_modes_17_to_64_rows():
                  (17, 4096, 4096, False), (32, 2048, 2048, False), (24, 4096, 512, False),
                  (32, 512, 512, False), (24, 2048, 1001, False), (33, 4096, 4096, False),
                  (64, 4096, 4096, True), (48, 4096, 14336, True), (24, 3584, 18944, True),
-                 (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 512, 512, True)]]
+                 (32, 14336, 4096, True), (24, 8192, 8192, True), (64, 1024, 512, True)]]
+    cases += [(dict(M=M, K=14336, N=4096, s_dtype="float32"), M > 21) for M in (17, 20, 26)]
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert lines and lines[0].startswith("woq prefill") == prefill, (call, lines)
 
@@ -69,18 +70,50 @@ def test_gate_up_large_tiles_or_two_steps():
         assert any(l.endswith(", gate_up") for l in lines) == merged, (call, lines)
 
 
-# short K at up to 64 rows: the synchronous kernel (it prints no launch line),
-# the large tiles past its limits
+# short K at up to 64 rows: the synchronous kernel (it prints no launch line) up to
+# a limit that grows with the rows, fp32 scales, columns that are not whole quads and
+# long post-ops; the large tiles past it
 def test_short_k_kernel():
-    cases = [(dict(M=M, K=K, N=256, **kind), prefill)
-             for kind, limit in ((dict(gs=32), 320), (dict(gs=64), 320),
-                                 (dict(gs=32, zp="int8"), 256), (dict(gs=64, s_dtype="float32"), 256))
-             for M, K, prefill in [(1, 64, False), (16, 192, False), (64, 192, False),
-                                   (64, 320, limit < 320), (16, 320, limit < 320),
-                                   (16, 448, True), (65, 64, True)]]
+    limits = [(dict(gs=32), 256, 320, 384), (dict(gs=64), 256, 320, 384), (dict(gs=64), 261, 512, 704),
+              (dict(gs=32, zp="int8"), 256, 256, 256), (dict(gs=32, zp="uint8"), 261, 320, 512),
+              (dict(gs=64, s_dtype="float32"), 256, 704, 704),
+              (dict(gs=64, s_dtype="float32", zp="int8"), 1001, 704, 704),
+              (dict(gs=64, post=["mul"]), 256, 320, 384), (dict(gs=64, post=["mul", "add"]), 256, 512, 704),
+              (dict(gs=64, post=["gelu_erf"]), 256, 512, 704),
+              (dict(gs=32, post=["silu", "mul"]), 261, 640, 704),
+              (dict(gs=64, zp="int8", post=["tanh"]), 256, 256, 576)]
+    cases = [(dict(M=M, K=K, N=N, **kind), K > (few if M <= 32 else many))
+             for kind, N, few, many in limits
+             for M in (1, 16, 17, 32, 33, 64) for K in (64, 192, 320, 448, 576, 704, 832)]
+    cases += [(dict(M=65, K=64, N=256, gs=64), True), (dict(M=65, K=704, N=261, gs=64), True)]
     for (call, prefill), (status, lines) in zip(cases, plans([c for c, _ in cases])):
         assert any(l.startswith("woq prefill") for l in lines) == prefill, (call, lines)
         assert prefill or not lines, (call, lines)
+
+
+# many columns of a short K past 32 rows: not the stream kernel, which reads x again
+# for every 16 of them; fewer columns, or a longer K, stay
+def test_short_k_many_columns():
+    cases = [(dict(M=M, K=K, N=N, **kind), stream)
+             for kind in (dict(gs=64), dict(gs=128, zp="int8"))
+             for M, K, N, stream in [(48, 640, 28672, False), (64, 384, 28672, False),
+                                     (48, 640, 12288, True), (24, 640, 28672, True),
+                                     (48, 1408, 28672, True)]]
+    for (call, stream), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert any(l.startswith("woq stream") for l in lines) == stream, (call, lines)
+
+
+# K of three phases with post-ops at 64 rows: zero points and small groups leave the
+# wide kernel for the large tiles
+def test_short_k_wide_kernel():
+    cases = [(dict(M=M, K=K, N=8192, post=post, **kind), wide)
+             for kind in (dict(gs=32), dict(gs=128, zp="int8"))
+             for M, K, post, wide in [(64, 768, ["mul", "add"], False), (64, 768, ["relu"], False),
+                                      (64, 768, [], True),
+                                      (64, 1024, ["add"], True)]]
+    cases += [(dict(M=64, K=768, N=8192, post=["add"]), True)]
+    for (call, wide), (status, lines) in zip(cases, plans([c for c, _ in cases])):
+        assert lines and lines[0].startswith("woq wide" if wide else "woq prefill"), (call, lines)
 
 
 # merged gate_up without its workspace: taken by the decode kernels' one launch

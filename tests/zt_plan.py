@@ -12,8 +12,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 
 def plans(calls, **knobs):
     """calls: dicts of M, K, N and optionally gs (scale group, default 128; 0:
-    per channel), zp and s_dtype ("int8", "float32", ..), gate_up, and workspace
-    (bytes; default what the size function asks for).  Returns one (status,
+    per channel), zp and s_dtype ("int8", "float32", ..), gate_up, post (names of
+    post-ops), and workspace (bytes; default what the size function asks for).  Returns one (status,
     [launch lines]) per call; knobs are ZT_ tuning knobs."""
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ZT_WOQ_DEBUG="1", **knobs)
     p = subprocess.run([sys.executable, os.path.abspath(__file__)], input=json.dumps(calls),
@@ -50,11 +50,16 @@ def _main():
         ws = c.get("workspace", size(M, K, N, G))
         head = (ptr, 1, M, K, K, ptr, N, ctypes.c_void_p(c.get("scales", 1 << 20)), s_dt, G,
                 ptr if zp else None, dt(zp) if zp else -1, None, -1)
+        post = C.PostOps(count=len(c.get("post", ())))
+        for i, name in enumerate(c.get("post", ())):
+            post.ids[i] = C.PO[name]
+            # (binary operands: bf16 [M, N], in the order of their ops)
+            post.bufs[i], post.buf_dtypes[i], post.buf_ld[i] = ptr.value, 1, N
         print("[call]", file=sys.stderr, flush=True)
         if gu:
             rc = L.zt_woq_linear_gate_up(*head, ptr, 1, N // 2, ptr if ws else None, ws, None)
         else:
-            rc = L.zt_woq_linear(*head, None, ptr, 1, N, ptr if ws else None, ws, None)
+            rc = L.zt_woq_linear(*head, ctypes.byref(post), ptr, 1, N, ptr if ws else None, ws, None)
         print("[end]", L.zt_last_error_string().decode() if rc else "ok", file=sys.stderr, flush=True)
 
 

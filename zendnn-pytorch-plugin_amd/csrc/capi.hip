@@ -339,7 +339,12 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
 
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   zt::WidePlan wp;
-  const bool wide = zt::woq_wide_ok(a, &wp);
+  bool wide = zt::woq_wide_ok(a, &wp);
+  // (three phases run as four, and its epilogue takes post-ops element by element: 8192 x
+  // 768 in groups of 32 with a mul and an add at 64 rows 28.4 us, 19.7 synchronous)
+  const bool short_wide = wide && M > 2 * kWoqRowBlock && K > 512 && K <= 768 && a.post.count &&
+                          (zp || (G > 1 && K / G < 128)) && !zt::knob(zt::kKnobWoqForceKernel);
+  if (short_wide) wide = false;
   const size_t need = wide ? zt::woq_wide_workspace(wp, M, N) : 0;
   const bool room = !need || (workspace && workspace_bytes >= need);
   // (zero points and groups of 32 / 64 have other kernels to go to without it)
@@ -353,8 +358,12 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
     const char *f = zt::knob(zt::kKnobWoqForceKernel);
     hipError_t err = hipSuccess;
     // (many columns of a short K re-read x for every row tile: 28672 x 256 at
-    // M = 32 / 64 8.7 / 13.1 us on the stream kernel, 7.6 / 8.1 on the synchronous one)
-    const bool rereads = !f && M > kWoqRowBlock && M * N > (1 << 19) && zt::woq_short_k(a);
+    // M = 32 / 64 8.7 / 13.1 us on the stream kernel, 7.6 / 8.1 on the synchronous one,
+    // 28672 x 640 with zero points at 33 to 64 rows 25.5 against 14.2 on the large tiles; 12288
+    // columns there 10.3 on the stream kernel, 12.5)
+    const bool rereads = !f && M > kWoqRowBlock &&
+                         ((M * N > (1 << 19) && K <= (zp ? 256 : 320)) ||
+                          (M * N >= 7 << 17 && K <= 768) || short_wide);
     if ((!f || !std::strcmp(f, "decode")) && !rereads && zt::woq_try_group_stream(a, s, &err))
       return hip_status(err, op);
   }
@@ -365,10 +374,14 @@ int zt_woq_linear(const void *x, int32_t x_dtype, int64_t M, int64_t K,
   if (M > kWoqRowBlock && M <= kWoqRowBlockMax && (zp || scales_dtype == ZT_DT_F32) &&
       !zt::knob(zt::kKnobWoqForceKernel) && !zt::knob(zt::kKnobWoqStream) &&
       zt::woq_prefill_ok(a)) {
-    if (zt::woq_short_k(a))
+    // (a short K: past 256 only where the blocks do not run or fp32 scales make
+    // three or four of them, 512 x 512 at M = 33 13.7 us in blocks, 11.5 synchronous)
+    const bool blocks = woq_use_row_blocks(a);
+    if (zt::woq_short_k(a) &&
+        (!blocks || K <= 256 || (M > 2 * kWoqRowBlock && scales_dtype == ZT_DT_F32)))
       return hip_status(zt::launch_woq_gemm(a, s, workspace, workspace_bytes), op);
     if (zt::woq_prefill_workspace(M, N, K) <= (workspace ? workspace_bytes : 0) &&
-        (!woq_use_row_blocks(a) || zt::woq_prefill_beats_row_blocks(a)))
+        (!blocks || zt::woq_prefill_beats_row_blocks(a)))
       return hip_status(zt::launch_woq_prefill(a, false, workspace, workspace_bytes, s), op);
   }
   if (woq_use_row_blocks(a)) {

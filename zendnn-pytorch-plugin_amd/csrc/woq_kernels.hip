@@ -2850,13 +2850,24 @@ size_t woq_gemm_workspace(int64_t M, int64_t N, int64_t K) {
 }
 
 // Up to 64 rows of a few steps of K the synchronous kernel's short prologue
-// wins over the large tiles' whole row tile (graph replays, 16 / 64 rows of 1024
-// columns: K = 64 3.8 / 4.2 us against 5.2 / 6.4, 256 6.0 / 6.7 against 6.8, 320 6.9 /
-// 7.6 against 7.3 / 8.4, 384 7.7 against 7.8; zero points and fp32 scales, which
-// it dequantises by two operations, K = 192 6.2 / 6.8 against 6.7 / 7.9, 256 7.4 against
-// 7.3, 320 8.6 against 7.9)
+// wins over the large tiles' whole row tile, which splits K only from 768 on (there they
+// are ahead by a third).  The lines lie where graph replays over 64 to 28672 columns cross
+// (synchronous / large tiles, us):
+//  * signed weights: 16 rows 320 6.9 / 7.3, 448 8.7 / 8.1; 64 rows 384 8.6 / 9.1, 448 9.4 / 9.4
+//  * two post-ops, or a function past relu, cost the large tiles 1 to 2 us more at up to 32 rows
+//    (448 9.6 / 10.5, 576 11.3 / 11.3) and 3 to 5 past them (704 ahead by 5 to 24 %)
+//  * columns that are not whole quads, stored one by one, likewise (1001 columns: 512 11.0 /
+//    11.2, past 32 rows 576 11.2 / 13.7, 704 ahead by up to 14 %)
+//  * zero points take the synchronous kernel two operations a weight: 256 7.4 / 7.3, 1001
+//    columns past 32 rows 448 11.9 / 13.4, 512 13.2 / 13.2
+//  * fp32 scales, the large tiles' slowest mode: 320 8.1 / 9.6, 704 14.7 / 14.9, 768 15.8 / 11.3
 bool woq_short_k(const WoqArgs &a) {
-  return a.M <= 64 && a.K <= (a.zp || a.s_dt == ZT_DT_F32 ? 256 : 320);
+  if (a.M > 64) return false;
+  const bool ragged = a.N % 4 != 0, many = a.M > 32, post = long_post_ops(a.post);
+  if (a.s_dt == ZT_DT_F32) return a.K <= 704;
+  if (a.zp)
+    return a.K <= (!many ? (ragged ? 320 : 256) : post ? (ragged ? 704 : 576) : ragged ? 512 : 256);
+  return a.K <= (!many ? (ragged ? (post ? 640 : 512) : post ? 512 : 320) : post || ragged ? 704 : 384);
 }
 
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s) {

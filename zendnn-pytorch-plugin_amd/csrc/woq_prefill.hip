@@ -495,17 +495,25 @@ PrefillPlan woq_prefill_plan(int64_t M, int64_t N, int64_t K, bool gate_up) {
 
 // Both sides from graph replays at 17 to 64 rows of 28 shapes, 256 x 256 to
 // 28672 x 4096 (bf16 zero points; fp32 scales; 8-bit zero points where N % 4
-// keeps the wide kernel away).  The choice is the faster one, or within 2 %, at
-// 422 of 427 points; 17 x 4096 x 4096 took 22.3 / 23.6 us (zero points / fp32
-// scales) here against 14.4 / 13.0 in blocks, 64 x 4096 x 4096 24 / 25 against 31 /
-// 28, 24 x 18944 x 3584 35 / 40 against 70 / 54.
+// keeps the wide kernel away), those of fp32 scales fitted again over 18 shapes at 17
+// to 40 rows.  The choice is the faster one, or within 2 %, at 422 of 427 points of the
+// first and within 5 % at those of the second past K = 704; 17 x 4096 x 4096 took 22.3 / 23.6 us (zero points /
+// fp32 scales) here against 14.4 / 13.0 in blocks, 64 x 4096 x 4096 24 / 25 against 31 /
+// 28, 24 x 18944 x 3584 35 / 40 against 70 / 54, 20 x 4096 x 14336 with fp32 scales 44
+// against 39.
 bool woq_prefill_beats_row_blocks(const WoqArgs &a) {
-  const double plan = woq_prefill_plan(a.M, a.N, a.K, false).us;
+  const PrefillPlan p = woq_prefill_plan(a.M, a.N, a.K, false);
+  const double plan = p.us;
   const bool f32 = a.s_dt == ZT_DT_F32;
   // (the plan's constants are those of the two one-FMA dequantisations)
-  const double here = f32                                               ? 1.32 * plan + 0.7
+  const double here = f32                                               ? 1.35 * plan + 0.0002 * a.K
                       : a.zp_dt == ZT_DT_S8 || a.zp_dt == ZT_DT_U8 ? 0.9 * plan
                                                                         : 1.13 * plan + 1.6;
+  // (unsplit, in few waves: post-ops past one relu or operand, 5 us of 512 x 1000 at M =
+  // 48, and columns that are not whole quads and are stored one by one)
+  const double epilogue =
+      p.splits > 1 ? 0.0
+                   : (double)a.M * ((a.N % 4 ? 0.045 : 0.0) + (long_post_ops(a.post) ? 0.1 : 0.0));
   // a round of 256 row tiles of 16, x whole in LDS (stream kernel) or not
   const double k = (double)a.K;
   const double round =
@@ -514,7 +522,7 @@ bool woq_prefill_beats_row_blocks(const WoqArgs &a) {
           : (f32 ? 0.0014 : 0.0016) * k;
   const int64_t rounds = ((a.N + 15) / 16 + 255) / 256, blocks = (a.M + 15) / 16;
   const double last = 0.6 + 0.4 / 16 * (double)(a.M - 16 * (blocks - 1));
-  return here < (3.0 + rounds * round) * (blocks - 1 + last);
+  return here + epilogue < (3.0 + rounds * round) * (blocks - 1 + last);
 }
 
 size_t woq_prefill_workspace(int64_t M, int64_t N, int64_t K) {

@@ -56,6 +56,12 @@ hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s);
 // with less it runs unsplit.
 hipError_t launch_woq_gemm(const WoqArgs &a, hipStream_t s, void *workspace,
                            size_t workspace_bytes);
+// Whether the post-ops are two and more or hold a function past relu, which costs the
+// large tiles' few waves more than the smaller tiles' many.
+inline bool long_post_ops(const PostOps &p) {
+  return p.count > 1 || (p.count == 1 && p.ids[0] != ZT_PO_RELU && p.ids[0] != ZT_PO_ADD &&
+                         p.ids[0] != ZT_PO_MUL);
+}
 // Whether launch_woq_gemm takes its synchronous kernel for a short K.
 bool woq_short_k(const WoqArgs &a);
 // Large-tile prefill GEMM (woq_prefill.hip): whether it takes these
